@@ -1959,6 +1959,19 @@ int kmoe_kv_store(kmoe_ctx *c, const float *k, const float *v, int64_t s_rows, i
   return KMOE_OK;
 }
 
+// A prompt chunk's attention on the matrix cores, where its shape allows (*done).
+static int attention_rows(kmoe_ctx *c, const float *q, const uint16_t *k_cache, const uint16_t *v_cache,
+                          int64_t s_rows, int32_t n_head, int32_t n_kv, int32_t head_dim, int64_t pos0,
+                          const int32_t *pos_dev, int64_t n_ctx, float *out, bool *done) {
+  const hipError_t e = timed(c, "attention", [&]() {
+    return launch_attn_rows(c->stream, q, k_cache, v_cache, s_rows, n_head, n_kv, head_dim, pos0, pos_dev, n_ctx,
+                            out);
+  });
+  *done = e == hipSuccess;
+  if (e != hipErrorNotSupported) HIP_OK(c, e);
+  return KMOE_OK;
+}
+
 int kmoe_attention(kmoe_ctx *c, const float *q, const uint16_t *k_cache, const uint16_t *v_cache, int64_t s_rows,
                    int32_t n_head, int32_t n_kv, int32_t head_dim, int64_t pos0, const int32_t *pos_dev,
                    int64_t n_ctx, float *out) {
@@ -1973,6 +1986,9 @@ int kmoe_attention(kmoe_ctx *c, const float *q, const uint16_t *k_cache, const u
   if (s_rows == 0) return KMOE_OK;
   if (!q || !k_cache || !v_cache || !out) return fail(c, KMOE_E_INVALID, "null pointer");
   DeviceGuard g(c->device);
+  bool done = false;
+  rc = attention_rows(c, q, k_cache, v_cache, s_rows, n_head, n_kv, head_dim, pos0, pos_dev, n_ctx, out, &done);
+  if (rc || done) return rc;
   const int supers = attn_supers(pos_dev ? n_ctx : std::min(n_ctx, pos0 + s_rows));
   rc = ensure_aws(c, (size_t)s_rows * n_head, (size_t)attn_part_floats(s_rows, n_head, head_dim, supers) * 4);
   if (rc) return rc;
@@ -2008,15 +2024,22 @@ int kmoe_attention_matmul(kmoe_ctx *c, const float *q, const uint16_t *k_cache, 
     rc = check_quant_shape(c, t, cols);
     if (rc) return rc;
   }
-  const int supers = attn_supers(pos_dev ? n_ctx : std::min(n_ctx, pos0 + s_rows));
-  rc = ensure_aws(c, (size_t)s_rows * n_head, (size_t)attn_part_floats(s_rows, n_head, head_dim, supers) * 4);
-  if (rc) return rc;
   const int64_t pf = gemm_f32_part_floats(rows, cols, 1, s_rows, s_rows);
   size_t need = 0;
   carve_qrows(nullptr, s_rows, cols, &need, pf);
   rc = ensure_ws(c, need);
   if (rc) return rc;
   QRows qr = carve_qrows(c->ws, s_rows, cols, &need, pf);
+  bool done = false;
+  rc = attention_rows(c, q, k_cache, v_cache, s_rows, n_head, n_kv, head_dim, pos0, pos_dev, n_ctx, attn, &done);
+  if (rc) return rc;
+  if (done) {
+    if (rows == 0) return KMOE_OK;
+    return matmul_core(c, t, (const uint8_t *)w, rows, cols, attn, s_rows, out, qr);
+  }
+  const int supers = attn_supers(pos_dev ? n_ctx : std::min(n_ctx, pos0 + s_rows));
+  rc = ensure_aws(c, (size_t)s_rows * n_head, (size_t)attn_part_floats(s_rows, n_head, head_dim, supers) * 4);
+  if (rc) return rc;
   float *part = (float *)(c->aws + c->aws_counters);
   uint32_t *counters = (uint32_t *)c->aws;
   // Where the projection takes the integer path, the attention kernel writes

@@ -387,6 +387,12 @@ hipError_t launch_attention(hipStream_t st, const float *q, const uint16_t *kc, 
                             int nh, int nkv, int hd, int64_t pos0, const int32_t *pos_dev, int64_t n_ctx, int supers,
                             float *part, uint32_t *counters, float *out, int qt = 0, int8_t *xq = nullptr,
                             float *xd = nullptr, int32_t *xs = nullptr);
+// Prompt chunks of at least kAttnRowsMin rows on the matrix cores
+// (kmoe_attn_rows.hip): no workspace, no counters. hipErrorNotSupported below
+// that, for other head dims and for caches that are not 16-byte aligned.
+constexpr int64_t kAttnRowsMin = 16;
+hipError_t launch_attn_rows(hipStream_t st, const float *q, const uint16_t *kc, const uint16_t *vc, int64_t s_rows,
+                            int nh, int nkv, int hd, int64_t pos0, const int32_t *pos_dev, int64_t n_ctx, float *out);
 // RoPE of q (into q_out) and k, and the f16 store of k and v into the caches.
 hipError_t launch_rope_kv(hipStream_t st, const float *q, const float *k, const float *v, int64_t s_rows, int nh,
                           int nkv, int hd, int rd, int64_t pos0, const int32_t *pos_dev, const float *inv_freq,

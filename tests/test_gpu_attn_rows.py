@@ -1,0 +1,73 @@
+"""Prompt-chunk attention on the matrix cores (kmoe_attn_rows.hip) against the oracle."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _run(ctx, q, kc, vc, nh, nkv, hd, pos0, n_ctx, pos_dev=None):
+    import torch
+
+    d = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    return ctx.attention(d(q), d(kc.view(np.int16)), d(vc.view(np.int16)), nh, nkv, hd, pos0, n_ctx,
+                         pos_dev=pos_dev).cpu().numpy()
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from kestrel_amd.kmoe import Context
+
+    c = Context(0)
+    yield c
+    c.close()
+
+
+# one row tile and its edges (16, 32, 33), ragged key blocks, fewer positions
+# than a block, both wave counts (8 from 257 positions on a small grid), head
+# dims, query groups, heads that do not divide the XCDs
+@pytest.mark.parametrize("nh,nkv,hd,S,pos0", [(4, 4, 128, 16, 0), (4, 1, 64, 16, 3), (3, 1, 128, 32, 0),
+                                              (8, 2, 64, 33, 31), (2, 2, 128, 31, 226), (2, 1, 128, 40, 230),
+                                              (6, 2, 64, 70, 500), (32, 4, 64, 300, 9), (16, 16, 128, 530, 17)])
+def test_rows_match_oracle(ctx, nh, nkv, hd, S, pos0):
+    import torch
+    from oracle import pyoracle as orc
+
+    rng = np.random.default_rng(nh + S + pos0)
+    n_ctx = pos0 + S  # the cache ends with the last row's position
+    kc = orc.f16_store(rng.standard_normal((n_ctx, nkv * hd)) * 2)
+    vc = orc.f16_store(rng.standard_normal((n_ctx, nkv * hd)))
+    q = rng.standard_normal((S, nh * hd)).astype(np.float32)
+    q *= np.exp2(rng.integers(-20, 3, size=(S, 1))).astype(np.float32)  # rows of very different size
+    ref = orc.attention(q, kc, vc, nh, nkv, hd, pos0)
+    got = _run(ctx, q, kc, vc, nh, nkv, hd, pos0, n_ctx)
+    # the bound of the other attention kernels: f32 scores and sums in another order
+    assert np.abs(got - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+    pos = torch.tensor([pos0], dtype=torch.int32).cuda()
+    assert np.array_equal(got, _run(ctx, q, kc, vc, nh, nkv, hd, 0, n_ctx, pos_dev=pos))
+
+
+def test_values_that_are_not_finite_stay_in_the_rows_that_see_them(ctx):
+    """A cached V of inf or NaN (f16 overflow) reaches the rows at and after its
+    position, in its own head dim, and no earlier row of the same tile; huge q
+    rows give NaN where the oracle does."""
+    from oracle import pyoracle as orc
+
+    rng = np.random.default_rng(3)
+    nh, nkv, hd, S, pos0 = 4, 2, 128, 75, 20
+    n = pos0 + S
+    kc = orc.f16_store(rng.standard_normal((n, nkv * hd)))
+    v = rng.standard_normal((n, nkv * hd)).astype(np.float32)
+    v[45, 7] = np.inf
+    v[46, 7 + hd] = -np.inf
+    v[70, 100] = np.nan
+    v[94, 3] = np.inf
+    vc = v.astype(np.float16).view(np.uint16)
+    q = rng.standard_normal((S, nh * hd)).astype(np.float32)
+    q[30, :hd] = np.inf
+    with np.errstate(all="ignore"):
+        ref = orc.attention(q, kc, vc, nh, nkv, hd, pos0)
+    got = _run(ctx, q, kc, vc, nh, nkv, hd, pos0, n)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
+    f = np.isfinite(ref)
+    assert np.isinf(ref).any() and f.mean() > 0.9 and np.abs(got[f] - ref[f]).max() <= 1e-5 * max(1.0, np.abs(ref[f]).max())
