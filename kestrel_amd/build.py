@@ -40,6 +40,7 @@ FLAGS = [
 # VGPRs, where their scale epilogue reads them without AGPR copies.
 FILE_FLAGS = {
     "kmoe_mfma.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+    "kmoe_f16gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
 }
 
 

@@ -107,6 +107,25 @@ static std::mutex g_scratch_mu;
 // Device completion counters per context (words used by the decode router).
 constexpr int kCounterWords = 64;
 constexpr int kNormDone = 1;  // the decode router's residual writer (kmoe_norm_moe_ffn)
+// Where the f32 regime takes the f16 matrix cores (kmoe_f16gemm.hip). A
+// work-group there walks all columns in stages of one memory round trip each,
+// so a product that does not fill the chip costs that chain whatever its
+// size, while the kernels for few rows shrink with it. Measured (us, those ->
+// f16), one matrix: Q4_K 4096x4096 64 rows 28 -> 39, 96 rows 42 -> 40, 512
+// rows 184 -> 74; 2048x2816 128 rows 21 -> 26, 256 rows 50 -> 28; Q6_K
+// 4096x4096 16 rows 49 -> 66, 24 rows 70 -> 66, 128 rows 312 -> 69; Q8_0
+// 2048x2816 24 rows 40 -> 43, 48 rows 68 -> 43.
+bool f16_plain(int t, int64_t rows, int64_t s_rows) {
+  return t == KMOE_Q4_K ? s_rows >= 24 && s_rows * rows >= 390000 : s_rows >= 4 && s_rows * rows >= 90000;
+}
+// Expert layers (whole layer, us): Mixtral shape 48 tokens 411 -> 595, 64
+// tokens 656 -> 600, 512 tokens 3596 -> 1195; with Q6_K down 64 tokens 798 ->
+// 947, 96 tokens 963 -> 948; Qwen3 shape 16 tokens 85 -> 109, 96 tokens 248 ->
+// 140, 1777 tokens 2067 -> 702; DeepSeek-V2-Lite shape 32 tokens 255 -> 282,
+// 64 tokens 378 -> 355, 203 tokens 831 -> 356.
+bool f16_experts(int t, int64_t d, int64_t F, int64_t slots) {
+  return slots * F >= (t == KMOE_Q6_K ? 600000 : 300000) * (d + F) / d;
+}
 constexpr int kFewRows = 3;   // decode batches over narrow rows: experts of 1..3 rows take launch_few_int
 
 struct kmoe_ctx {
@@ -497,14 +516,54 @@ struct QRows {
   int32_t *s;
   float *part;
   int64_t part_floats;
+  F16Rows xf;  // the f32 regime's activation pieces, over the same bytes (planes null: no room for them)
 };
 QRows carve_qrows(uint8_t *base, int64_t s_rows, int64_t cols, size_t *total, int64_t part_floats = 0) {
   Carver cv{base};
   QRows r{cv.take<int8_t>(s_rows * cols), cv.take<float>(s_rows * (cols / 32)), cv.take<int32_t>(s_rows * (cols / 16)),
-          nullptr, part_floats};
+          nullptr, part_floats, F16Rows{}};
   r.part = part_floats > 0 ? cv.take<float>(part_floats) : nullptr;
   *total = cv.off;
   return r;
+}
+
+// Activation pieces of the f16 matrix-core path for [s_rows, cols] (cols
+// rounded up to 128), and the bytes they take.
+F16Rows carve_f16(uint8_t *base, int64_t s_rows, int64_t cols, size_t *total) {
+  Carver cv{base};
+  const int64_t kp = (cols + 127) / 128 * 128;
+  F16Rows r;
+  r.planes = cv.take<uint16_t>(s_rows * 2 * kp);
+  r.sums = cv.take<uint16_t>(s_rows * kp / 16);
+  r.sums_stride = kp / 8;
+  r.ex = cv.take<int32_t>(s_rows);
+  *total = cv.off;
+  return r;
+}
+
+// The scratch of one quant::matmul in the workspace: `need` bytes that it must
+// have (int8 rows, partial sums, more behind them) and, where the f16 matrix
+// cores can take the f32 regime, the activation pieces over the same bytes.
+// Those are left out (and the other f32 kernels run) where only they would
+// push the workspace past the VRAM budget, or grow it inside a graph capture.
+int matmul_ws(kmoe_ctx *c, int t, int64_t rows, int64_t s_rows, int64_t cols, int64_t part_floats, size_t need, QRows *qr) {
+  size_t f16 = 0;
+  if (f16_plain(t, rows, s_rows) && f16_gemm_supported(t, rows, cols, s_rows)) carve_f16(nullptr, s_rows, cols, &f16);
+  size_t want = f16 > need ? f16 : need;
+  if (want > need && want > c->ws_size) {
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) (void)hipGetLastError();
+    if (cap != hipStreamCaptureStatusNone ||
+        c->vram_reserved - c->ws_size + align_up(want + want / 4) > c->vram_limit)
+      want = need;
+  }
+  int rc = ensure_ws(c, want);
+  if (rc && want > need) rc = ensure_ws(c, need);
+  if (rc) return rc;
+  size_t n = 0;
+  *qr = carve_qrows(c->ws, s_rows, cols, &n, part_floats);
+  if (f16 && f16 <= c->ws_size) qr->xf = carve_f16(c->ws, s_rows, cols, &n);
+  return KMOE_OK;
 }
 
 // The f32 path's partial sums for the shared expert's three products.
@@ -539,6 +598,18 @@ int matmul_core(kmoe_ctx *c, int t, const uint8_t *w, int64_t rows, int64_t cols
     return KMOE_OK;
   }
   if (!int_path(c->regime, s_rows)) {
+    // the f16 matrix cores, where the activations' pieces have room
+    if (qr.xf.planes) {
+      F16Rows xf = qr.xf;
+      if (t != KMOE_Q4_K) xf.sums = nullptr;
+      hipError_t e = timed(c, "split_f16", [&]() { return launch_split_f16(c->stream, x, s_rows, cols, xf); });
+      if (e == hipSuccess)
+        e = timed(c, "f16_gemm", [&]() {
+          return launch_f16_gemm_plain(c->stream, t, w, rows, cols, xf, s_rows, out);
+        });
+      if (e == hipSuccess) return KMOE_OK;
+      if (e != hipErrorNotSupported) HIP_OK(c, e);
+    }
     // Q4_K rows: the bf16-split kernel (exact products on the bf16 matrix
     // cores); other types, or unaligned buffers, the fp32 GEMM
     if (t == KMOE_Q4_K) {
@@ -854,10 +925,9 @@ int kmoe_matmul(kmoe_ctx *c, int t, const void *w, size_t w_len, int64_t rows, i
   carve_qrows(nullptr, s_rows, cols, &need, pf);
   const size_t wf_off = need;
   if (staged) need = wf_off + align_up((size_t)rows * (size_t)cols * 4);
-  int rc = ensure_ws(c, need);
+  QRows qr{};
+  int rc = matmul_ws(c, t, rows, s_rows, cols, pf, need, &qr);
   if (rc) return rc;
-  size_t qn = 0;
-  QRows qr = carve_qrows(c->ws, s_rows, cols, &qn, pf);
   return matmul_core(c, t, (const uint8_t *)w, rows, cols, x, s_rows, out, qr,
                      staged ? (float *)(c->ws + wf_off) : nullptr);
 }
@@ -1429,6 +1499,7 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
   }
 
   const int gt = D.gate_type, dt = D.down_type;
+  bool sh_gs_done = false;  // the shared expert's SwiGLU rows are in sh_gs (f32 regime)
   {
   // route (transformer.rs:474-496) and dispatch (transformer.rs:525-531). With
   // s_rows < 4 one fused work-group also quantizes x for the int8 path.
@@ -1617,9 +1688,38 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
   // up in one launch; other row types take the staged GEMM.
   const int f32_lo = regime == KMOE_REGIME_EXACT ? 1 : 4;
   const int f32_hi = (int)S;
+  // The f16 matrix cores: x's pieces lie where y will (dead until the down
+  // product), their sums and exponents where h's int8 sums and scales will.
+  F16Rows xf;
+  bool xf_done = false;
   if (any_f32) {
+    const auto &SH = L->sh;
+    const bool sh_q4 = SH.on && !int_path(regime, S) && SH.type[0] == KMOE_Q4_K && SH.type[1] == KMOE_Q4_K;
     int f32_done = 0;  // experts with f32_lo..f32_done rows are done
-    if (gt == KMOE_Q4_K && L->tiled[0] && L->tiled[1] && f32_hi >= f32_lo) {
+    if (f16_experts(gt, d, F, slots) && f16_gemm_supported(gt, F, d, slots) && d % 128 == 0 && d <= 2 * k * F && k * F >= 32) {
+      xf.planes = (uint16_t *)w.y;
+      xf.sums = gt == KMOE_Q4_K || sh_q4 ? (uint16_t *)w.hs : nullptr;
+      xf.sums_stride = d / 8;
+      xf.ex = (int32_t *)w.hd;
+      const hipError_t e = timed(c, "split_f16", [&]() { return launch_split_f16(st, h, S, d, xf); });
+      if (e == hipSuccess) xf_done = true;
+      else if (e != hipErrorNotSupported) HIP_OK(c, e);
+    }
+    if (xf_done) {
+      hipError_t e = timed(c, "moe_gate_up_f16", [&]() {
+        return launch_f16_gemm(st, 0, gt, tier, F, d, rt, (int)E, max_active, slots, f32_lo, f32_hi, xf, w.h);
+      });
+      if (e == hipSuccess) f32_done = f32_hi;
+      else if (e != hipErrorNotSupported) HIP_OK(c, e);
+      if (sh_q4) {  // the shared expert's front reads the same pieces
+        e = timed(c, "shared_gate_up_f16", [&]() {
+          return launch_f16_gemm_plain(st, KMOE_Q4_K, SH.arena + SH.off[0], Fs, d, xf, S, sh_gs, SH.arena + SH.off[1]);
+        });
+        if (e == hipSuccess) sh_gs_done = true;
+        else if (e != hipErrorNotSupported) HIP_OK(c, e);
+      }
+    }
+    if (f32_done == 0 && gt == KMOE_Q4_K && L->tiled[0] && L->tiled[1] && f32_hi >= f32_lo) {
       const hipError_t e = timed(c, "moe_gate_up_f32_rows", [&]() {
         return launch_f32_rows(st, 0, gt, tier, F, d, rt, regime, max_active, slots, f32_lo, f32_hi, h, w.h);
       });
@@ -1668,7 +1768,27 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
   }
   if (any_f32) {
     int f32_done = 0;
-    if (dt == KMOE_Q4_K && L->tiled[2] && f32_hi >= f32_lo) {
+    // h's pieces in place; their sums and exponents in the slots' int8 sums and
+    // scales, which the f32 regime's slots do not use
+    if (f16_experts(dt, d, F, slots) && f16_gemm_supported(dt, d, F, slots) && F % 128 == 0) {
+      F16Rows hf;
+      hf.planes = (uint16_t *)w.h;
+      hf.sums = dt == KMOE_Q4_K ? (uint16_t *)w.hs : nullptr;
+      hf.sums_stride = F / 16 * 4;
+      hf.ex = (int32_t *)w.hd;
+      hf.ex_stride = F / 32;
+      hipError_t e = timed(c, "split_slots_f16", [&]() {
+        return launch_split_f16(st, w.h, slots, F, hf, &rt, w.idx, f32_lo);
+      });
+      if (e == hipSuccess) {  // from here on these slots' h is pieces only
+        LAUNCH(c, "moe_down_f16",
+               launch_f16_gemm(st, 1, dt, tier, d, F, rt, (int)E, max_active, slots, f32_lo, f32_hi, hf, w.y));
+        f32_done = f32_hi;
+      } else if (e != hipErrorNotSupported) {
+        HIP_OK(c, e);
+      }
+    }
+    if (f32_done == 0 && dt == KMOE_Q4_K && L->tiled[2] && f32_hi >= f32_lo) {
       const hipError_t e = timed(c, "moe_down_f32_rows", [&]() {
         return launch_f32_rows(st, 1, dt, tier, d, F, rt, regime, max_active, slots, f32_lo, f32_hi, w.h, w.y);
       });
@@ -1729,8 +1849,8 @@ done:
       goto shared_done;
     }
     // f32 regime, Q4_K gate and up: both products and SwiGLU in one launch
-    hipError_t ef = hipErrorNotSupported;
-    if (!int_path(c->regime, S) && SH.type[0] == KMOE_Q4_K && SH.type[1] == KMOE_Q4_K)
+    hipError_t ef = sh_gs_done ? hipSuccess : hipErrorNotSupported;
+    if (!sh_gs_done && !int_path(c->regime, S) && SH.type[0] == KMOE_Q4_K && SH.type[1] == KMOE_Q4_K)
       ef = timed(c, "shared_gate_up_f32", [&]() {
         return launch_f32_rows_plain(st, KMOE_Q4_K, SH.arena + SH.off[0], Fs, d, h, S, gs, SH.arena + SH.off[1]);
       });
@@ -1742,7 +1862,26 @@ done:
       if (rc) return rc;
       LAUNCH(c, "shared_swiglu", launch_swiglu(st, gs, us, S * Fs));
     }
-    rc = matmul_core(c, SH.type[2], SH.arena + SH.off[2], d, Fs, gs, S, ys, qr);
+    bool ys_done = false;
+    if (!int_path(regime, S) && f16_plain(t2, d, S) && f16_gemm_supported(t2, d, Fs, S) && Fs % 128 == 0) {
+      // the SwiGLU rows' pieces in place, their sums and exponents in the int8 scratch
+      F16Rows gf;
+      gf.planes = (uint16_t *)gs;
+      gf.sums = t2 == KMOE_Q4_K ? (uint16_t *)qr.q : nullptr;
+      gf.sums_stride = Fs / 8;
+      gf.ex = qr.s;
+      const uintptr_t al = t2 == KMOE_Q4_K ? 15u : 1u;
+      hipError_t e = hipErrorNotSupported;
+      if (((uintptr_t)(SH.arena + SH.off[2]) & al) == 0)
+        e = timed(c, "split_f16", [&]() { return launch_split_f16(st, gs, S, Fs, gf); });
+      if (e == hipSuccess) {
+        LAUNCH(c, "shared_down_f16", launch_f16_gemm_plain(st, t2, SH.arena + SH.off[2], d, Fs, gf, S, ys));
+        ys_done = true;
+      } else if (e != hipErrorNotSupported) {
+        HIP_OK(c, e);
+      }
+    }
+    if (!ys_done) rc = matmul_core(c, SH.type[2], SH.arena + SH.off[2], d, Fs, gs, S, ys, qr);
     if (rc) return rc;
     if (SH.gate_ok) LAUNCH(c, "shared_gate", launch_router_logits(st, SH.gate_inp, 1, d, h, S, gl, true));
     LAUNCH(c, "shared_add", launch_shared_add(st, out, ys, SH.gate_ok ? gl : nullptr, S, d));
@@ -1906,9 +2045,9 @@ int kmoe_norm_matmul(kmoe_ctx *c, float *x, const float *y, const float *norm_w,
   const int64_t pf = gemm_f32_part_floats(rows, cols, 1, s_rows, s_rows);
   size_t need = 0;
   carve_qrows(nullptr, s_rows, cols, &need, pf);
-  int rc = ensure_ws(c, need);
+  QRows qr{};
+  int rc = matmul_ws(c, t, rows, s_rows, cols, pf, need, &qr);
   if (rc) return rc;
-  QRows qr = carve_qrows(c->ws, s_rows, cols, &need, pf);
   if (t != KMOE_F32 && int_path(c->regime, s_rows) && rows > 0) {
     hipError_t e = timed(c, "rmsnorm_quant", [&]() {
       return launch_rmsnorm_quant(c->stream, x, y, norm_w, s_rows, cols, eps, h, is_kq(t), qr.q, qr.d, qr.s);
@@ -2027,9 +2166,9 @@ int kmoe_attention_matmul(kmoe_ctx *c, const float *q, const uint16_t *k_cache, 
   const int64_t pf = gemm_f32_part_floats(rows, cols, 1, s_rows, s_rows);
   size_t need = 0;
   carve_qrows(nullptr, s_rows, cols, &need, pf);
-  rc = ensure_ws(c, need);
+  QRows qr{};
+  rc = matmul_ws(c, t, rows, s_rows, cols, pf, need, &qr);
   if (rc) return rc;
-  QRows qr = carve_qrows(c->ws, s_rows, cols, &need, pf);
   bool done = false;
   rc = attention_rows(c, q, k_cache, v_cache, s_rows, n_head, n_kv, head_dim, pos0, pos_dev, n_ctx, attn, &done);
   if (rc) return rc;

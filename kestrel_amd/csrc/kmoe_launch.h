@@ -261,6 +261,38 @@ hipError_t launch_f32_rows(hipStream_t st, int mode, int type, const ExpertTier 
                            const Routing &rt, int regime, int max_active, int64_t n_slots, int min_rows,
                            int max_rows, const float *x, float *out);
 
+// ---- the f32 regime for many rows on the f16 matrix cores (kmoe_f16gemm.hip):
+// Q4_K, Q6_K and Q8_0 rows against activation rows held as two f16 pieces.
+// Rows of pieces: planes [rows][2][cols rounded up to 128] f16 (16-byte
+// aligned), the scaling exponent of row r at ex[r * ex_stride], and for Q4_K
+// weights the 32-sums' pieces (32 bytes per 256 columns) at sums + r *
+// sums_stride bytes (16-byte aligned rows).
+struct F16Rows {
+  uint16_t *planes = nullptr;
+  uint16_t *sums = nullptr;
+  int64_t sums_stride = 0;
+  int32_t *ex = nullptr;
+  int64_t ex_stride = 1;
+};
+// Weights [rows, cols] of this type against n activation rows (slots).
+bool f16_gemm_supported(int type, int64_t rows, int64_t cols, int64_t n);
+// x [rows, cols] f32 (16-byte aligned) -> pieces. Rows of a multiple of 128
+// columns may convert in place (planes = x). sums null: no sums. With rt and
+// idx (the flat expert choice), rows are slots in dispatch order and only those
+// of experts with at least min_rows rows are converted.
+hipError_t launch_split_f16(hipStream_t st, const float *x, int64_t rows, int64_t cols, const F16Rows &o,
+                            const Routing *rt = nullptr, const uint32_t *idx = nullptr, int min_rows = 0);
+// Grouped, experts with min_rows..max_rows rows: mode 0 gate/up + SwiGLU (x:
+// the tokens' rows) into out [slots, rows], mode 1 down (x: the slots' rows).
+// hipErrorNotSupported (nothing launched) for other types or shapes.
+hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier &tier, int64_t rows, int64_t cols,
+                           const Routing &rt, int n_expert, int max_active, int64_t n_slots, int min_rows,
+                           int max_rows, const F16Rows &x, float *out);
+// Plain GGUF rows: out [s_rows, rows]; with w_up (Q4_K) SwiGLU(w . x, w_up . x).
+// hipErrorNotSupported for other types, shapes or alignments.
+hipError_t launch_f16_gemm_plain(hipStream_t st, int type, const uint8_t *w, int64_t rows, int64_t cols,
+                                 const F16Rows &x, int64_t s_rows, float *out, const uint8_t *w_up = nullptr);
+
 // ---- routing (kmoe_route.hip)
 // logits [S, E] = router [E, d] . x [S, d] in the reference's summation order
 // for s_rows (quant::matmul), or always in quant::dot order when qdot is set.

@@ -1,0 +1,140 @@
+"""The f32 regime on the f16 matrix cores (kmoe_f16gemm.hip): many activation
+rows against Q4_K, Q6_K and Q8_0 weights, plain and in expert layers."""
+import numpy as np
+import pytest
+
+from helpers import Q4_K, Q6_K, Q8_0, LayerSpec, random_blocks, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from kestrel_amd.kmoe import Context
+
+    c = Context(0)
+    c.profile_enable(True)
+    yield c
+    c.close()
+
+
+def _matmul(ctx, t, w, rows, cols, x):
+    import torch
+
+    n0 = ctx.profile_read("f16_gemm")[1]
+    out = ctx.matmul(t, torch.from_numpy(w).cuda(), rows, cols, torch.from_numpy(x).cuda()).cpu().numpy()
+    assert ctx.profile_read("f16_gemm")[1] == n0 + 1, "another kernel ran"
+    return out
+
+
+def _bound(t, w64, x, cols):
+    """Largest error of the sum of products: the pieces (2^-23 of each x, 2^-40
+    of the row's largest) and one fp32 rounding per 8 products of partial sums
+    no larger than sum |w x| (Q4_K: of the scale and the minimum term apart, at
+    most 8 times that for these blocks: |d sc q| + |dmin m| <= 7 * max |w| of
+    the sub-block, its rms at least max / 4)."""
+    a = np.abs(x).astype(np.float64)
+    s = a @ np.abs(w64).T + 2.0 ** -17 * a.max(1, keepdims=True) * np.abs(w64).sum(1)
+    return (cols / 8 + 8) * 2.0 ** -24 * s * (8 if t == Q4_K else 1)
+
+
+# edges of the row blocks (128, 256), of the 32-token tiles and 64-token blocks,
+# rows that end inside a 128-column stage (Q8_0), one and several superblocks,
+# one and two token tiles per work-group
+@pytest.mark.parametrize("t,rows,cols,S", [(Q4_K, 16390, 256, 24), (Q4_K, 4100, 512, 97), (Q4_K, 33000, 768, 64),
+                                           (Q4_K, 1500, 2048, 513), (Q8_0, 3000, 64, 31), (Q8_0, 2817, 1344, 33),
+                                           (Q8_0, 40001, 192, 65), (Q6_K, 22501, 256, 4), (Q6_K, 700, 768, 130),
+                                           (Q6_K, 33001, 512, 95)])
+def test_plain_rows(ctx, t, rows, cols, S):
+    from oracle import pyoracle as orc
+
+    w = random_blocks(t, rows, cols, seed=rows + cols)
+    rng = np.random.default_rng(S)
+    x = rng.standard_normal((S, cols)).astype(np.float32)
+    x *= np.exp2(rng.integers(-60, 60, size=(S, 1))).astype(np.float32)  # rows of very different size
+    x[1] = 0.0
+    x[2, 3::7] *= np.float32(2.0 ** -20)  # and small elements beside large ones
+    w64 = orc.dequant(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    ref = x.astype(np.float64) @ w64.T
+    got = _matmul(ctx, t, w, rows, cols, x)
+    assert np.all(np.abs(got - ref) <= _bound(t, w64, x, cols) + 1e-45)
+    n = np.linalg.norm(ref, axis=1)
+    assert np.all(np.linalg.norm(got - ref, axis=1) <= 1e-6 * n)
+
+
+@pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0])
+def test_values_that_are_not_finite_stay_in_their_row(ctx, t):
+    from oracle import pyoracle as orc
+
+    rows, cols, S = 6000, 512, 70
+    w = random_blocks(t, rows, cols, seed=3)
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((S, cols)).astype(np.float32)
+    x[5, 100] = np.inf
+    x[40, 3] = np.nan
+    x[69, 500] = -np.inf
+    x[7] *= np.float32(3e38 / np.abs(x[7]).max())  # the sums overflow
+    got = _matmul(ctx, t, w, rows, cols, x)
+    w64 = orc.dequant(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    fin = np.ones(S, bool)
+    fin[[5, 40, 69, 7]] = False
+    assert not np.isfinite(got[[5, 40, 69]]).any()
+    assert rel_l2(got[fin], x[fin].astype(np.float64) @ w64.T) < 1e-6
+    ref7 = (x[7].astype(np.float64) / 2.0 ** 20) @ w64.T
+    over, under = np.abs(ref7) > 3.5e38 / 2.0 ** 20, np.abs(ref7) < 3.3e38 / 2.0 ** 20
+    assert np.isinf(got[7][over]).all() and np.isfinite(got[7][under]).all()
+    assert np.array_equal(np.sign(got[7][over]), np.sign(ref7[over]))
+
+
+# ragged experts (Zipf: one of several hundred rows, some of none or below the
+# f32 regime's 4), in both f32 regimes; gate/up and down of every type
+@pytest.mark.parametrize("E,k,d,F,S,gt,dt,regime", [(9, 2, 512, 384, 701, Q4_K, Q8_0, 0),
+                                                    (70, 3, 256, 512, 900, Q4_K, Q4_K, 2),
+                                                    (6, 2, 256, 512, 1801, Q6_K, Q6_K, 0),
+                                                    (5, 1, 512, 256, 1801, Q8_0, Q4_K, 0)])
+def test_expert_layers(ctx, E, k, d, F, S, gt, dt, regime):
+    import torch
+    from oracle import pyoracle as orc
+
+    spec = LayerSpec(E, k, d, F, gt, seed=E + S, down_type=dt, zipf=1.3)
+    x = orc.normal(S, S * d).reshape(S, d) + np.float32(1.0)
+    spec.upload(ctx, E)
+    n0 = [ctx.profile_read(n)[1] for n in ("moe_gate_up_f16", "moe_down_f16")]
+    ctx.set_regime(regime)
+    try:
+        out = ctx.moe_ffn(E, torch.from_numpy(x).cuda()).cpu().numpy()
+    finally:
+        ctx.set_regime(0)
+    assert [ctx.profile_read(n)[1] for n in ("moe_gate_up_f16", "moe_down_f16")] == [n + 1 for n in n0]
+    layer = spec.oracle_layer()
+    idx = ctx.last_routing(S, k, E)[0].cpu().numpy().astype(np.uint32)
+    assert np.array_equal(idx, layer.route(x)[0])
+    cnt = np.bincount(idx.ravel(), minlength=E)
+    ref = layer.moe_ffn(x, regime)
+    big = cnt[idx].min(1) >= 4 if regime == 0 else np.ones(S, bool)  # tokens whose experts are all in the f32 regime
+    assert big.sum() > S // 2
+    assert rel_l2(out[big], ref[big]) < 3e-6
+    assert rel_l2(out, ref) < 1e-3
+
+
+def test_a_budget_without_room_for_the_pieces_keeps_the_other_kernels():
+    import torch
+    from kestrel_amd.kmoe import Context
+    from oracle import pyoracle as orc
+
+    rows, cols, S = 40000, 256, 600  # no partial sums: the pieces are the larger need
+    w = random_blocks(Q4_K, rows, cols, seed=8)
+    x = orc.normal(8, S * cols).reshape(S, cols)
+    c = Context(0)
+    c.profile_enable(True)
+    wd, xd = torch.from_numpy(w).cuda(), torch.from_numpy(x).cuda()
+    full = c.matmul(Q4_K, wd, rows, cols, xd).cpu().numpy()
+    used = c.vram_usage()[0]
+    c.close()
+    c = Context(0)
+    c.profile_enable(True)
+    c.vram_set_limit(used - 1)
+    tight = c.matmul(Q4_K, wd, rows, cols, xd).cpu().numpy()
+    assert c.profile_read("f16_gemm")[1] == 0 and c.profile_read("f32_rows_plain")[1] == 1
+    c.close()
+    assert rel_l2(full, tight) < 2e-6
