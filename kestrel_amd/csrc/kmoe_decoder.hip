@@ -340,7 +340,10 @@ __device__ __forceinline__ float attn_score(const float *qh, const uint4 (&kr)[H
   float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
   for (int j = 0; j < KV4; ++j) {
-    const uint32_t w4[4] = {kr[j].x, kr[j].y, kr[j].z, kr[j].w};
+    uint32_t w4[4] = {kr[j].x, kr[j].y, kr[j].z, kr[j].w};
+    // in order: q read and K converted as they are used (all of both at once,
+    // or converted outside a loop over heads, would take 256 registers more)
+    asm volatile("" : "+v"(w4[0]), "+v"(w4[1]), "+v"(w4[2]), "+v"(w4[3])::"memory");
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const float a0 = qh[8 * j + 2 * i] * f16_bits_to_f32(w4[i]);
@@ -368,7 +371,10 @@ __device__ __forceinline__ void attn_wv(const float *ws, const uint4 (&vp)[HD / 
     const int r = j * RPI + rc;
     const float w = ws[r];
     const bool live = r < np;
-    const uint32_t u[4] = {live ? vp[j].x : 0u, live ? vp[j].y : 0u, live ? vp[j].z : 0u, live ? vp[j].w : 0u};
+    uint32_t u[4] = {vp[j].x, vp[j].y, vp[j].z, vp[j].w};
+    asm volatile("" : "+v"(u[0]), "+v"(u[1]), "+v"(u[2]), "+v"(u[3]));  // as in attn_score
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = live ? u[i] : 0u;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       a[2 * i] = a[2 * i] + w * f16_bits_to_f32(u[i]);
@@ -411,12 +417,79 @@ __device__ __forceinline__ void attn_quant_group(const float *os, int group, int
   }
 }
 
+// The chunk partials of one head, handed over by other work-groups (agent
+// scope), merged by one wave in chunk order. Lane c holds chunk c's m and l and
+// its factor; the accumulators of 16 chunks are loaded at once, the first 16
+// before the factors are formed. What bounds a long row is this chain and how
+// many chunks are resident: eight chunks per round trip with m and l read
+// again for each, and one work-group per CU (f32 copies of K, V and q held in
+// 300 registers), took 38.5 us for one row of 16 heads of 128 at 3001
+// positions; this merge with three work-groups per CU 21 us (4096 positions
+// 49.6 -> 32.2; 8 rows of 16 heads over 4 at 1008 positions 25.0 -> 16.8).
+template <int HD>
+__device__ __forceinline__ void attn_merge(const float *pb, int nch, int lane, float *__restrict__ out, float *os) {
+  constexpr int DPL = HD / 64, PW = HD + 2, B = 16;
+  typedef float fv __attribute__((ext_vector_type(2)));
+  auto acc = [&](int c, float (&o)[DPL]) {
+    const float *p = pb + (int64_t)(c < nch ? c : nch - 1) * PW + 2 + lane * DPL;
+    if constexpr (DPL == 2) {  // PW is even: 8-byte aligned
+      const fv v = __builtin_bit_cast(fv, __hip_atomic_load((const uint64_t *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      o[0] = v.x;
+      o[1] = v.y;
+    } else {
+      o[0] = ld_agent(p);
+    }
+  };
+  float ov[B][DPL];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int j = 0; j < B; ++j) acc(c0 + j, ov[j]);
+  };
+  load(0);
+  float mv = lane < nch ? ld_agent(pb + (int64_t)lane * PW) : -INFINITY;
+  float lv = lane < nch ? ld_agent(pb + (int64_t)lane * PW + 1) : 0.0f;
+  float M = mv;
+  for (int c = 64 + lane; c < nch; c += 64) M = fmaxf(M, ld_agent(pb + (int64_t)c * PW));
+  M = group_max<64>(M);
+  float L = 0.0f, O[DPL];
+#pragma unroll
+  for (int i = 0; i < DPL; ++i) O[i] = 0.0f;
+  for (int c0 = 0; c0 < nch; c0 += B) {
+    if (c0 > 0) {
+      load(c0);
+      if (c0 % 64 == 0) {
+        mv = c0 + lane < nch ? ld_agent(pb + (int64_t)(c0 + lane) * PW) : -INFINITY;
+        lv = c0 + lane < nch ? ld_agent(pb + (int64_t)(c0 + lane) * PW + 1) : 0.0f;
+      }
+    }
+    const float f = expf(mv - M), lf = lv * f;
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+      if (c0 + j < nch) {
+        const int l = (c0 & 63) + j;
+        const float fc = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), l));
+        L += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, lf), l));
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) O[i] += ov[j][i] * fc;
+      }
+    }
+  }
+  const float inv = 1.0f / L;
+#pragma unroll
+  for (int i = 0; i < DPL; ++i) {
+    const float r = O[i] * inv;
+    out[lane * DPL + i] = r;
+    os[lane * DPL + i] = r;
+  }
+}
+
 // Work-group bid = (kv head g, query row s, chunk c) of 256 threads; wave w
 // takes query heads w, w + 4, ... of the group over the chunk, whose K rows the
 // work-group loads into its tile together. With one chunk the result is final;
 // otherwise every work-group of the row hands (m, l, acc) over with agent-scope
 // stores and a counter, and the last to arrive merges them and resets the
-// counter. LDS: Qs and Os [kMaxGroup][HD], Ws [4][64], one K tile.
+// counter. LDS: Qs and Os [kMaxGroup][HD] (Os may be Qs: a head's output is
+// written by the wave that read its q), Ws [4][64], one K tile.
 template <int HD>
 __device__ __forceinline__ void attn_batch(int64_t bid, const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                            const uint16_t *__restrict__ vc, int64_t s_rows, int nh, int nkv,
@@ -426,8 +499,7 @@ __device__ __forceinline__ void attn_batch(int64_t bid, const float *__restrict_
                                            int32_t *__restrict__ xs, float (*Qs)[HD], float (*Os)[HD],
                                            float (*Ws)[kAttnChunk], AttnKTile<HD> &Kt, uint32_t &last) {
   constexpr int KV4 = HD / 8;
-  constexpr int DPL = HD / 64;  // head dims per lane in the merge
-  constexpr int PW = HD + 2;    // one chunk partial: m, l, acc[HD]
+  constexpr int PW = HD + 2;  // one chunk partial: m, l, acc[HD]
   const int c = (int)(bid % nch_grid);
   const int64_t s = (bid / nch_grid) % s_rows;
   const int g = (int)(bid / nch_grid / s_rows);
@@ -515,49 +587,7 @@ __device__ __forceinline__ void attn_batch(int64_t bid, const float *__restrict_
   if (last != (uint32_t)(nch - 1)) return;
   for (int hh = wave; hh < group; hh += 4) {
     const int64_t h = (int64_t)g * group + hh;
-    const float *pb = part + (s * nh + h) * nch_grid * PW;
-    // the partials of 8 chunks at a time, every load issued before any use
-    constexpr int B = 8;
-    float M = -INFINITY;
-    for (int c0 = 0; c0 < nch; c0 += B) {
-      float mv[B];
-#pragma unroll
-      for (int j = 0; j < B; ++j) mv[j] = c0 + j < nch ? ld_agent(pb + (c0 + j) * PW) : -INFINITY;
-#pragma unroll
-      for (int j = 0; j < B; ++j) M = fmaxf(M, mv[j]);
-    }
-    float L = 0.0f, O[DPL];
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) O[i] = 0.0f;
-    for (int c0 = 0; c0 < nch; c0 += B) {
-      float mv[B], lv[B], ov[B][DPL];
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        if (c0 + j < nch) {
-          const float *pc = pb + (c0 + j) * PW;
-          mv[j] = ld_agent(pc);
-          lv[j] = ld_agent(pc + 1);
-#pragma unroll
-          for (int i = 0; i < DPL; ++i) ov[j][i] = ld_agent(pc + 2 + lane * DPL + i);
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < B; ++j) {
-        if (c0 + j < nch) {
-          const float f = expf(mv[j] - M);
-          L += lv[j] * f;
-#pragma unroll
-          for (int i = 0; i < DPL; ++i) O[i] += ov[j][i] * f;
-        }
-      }
-    }
-    const float inv = 1.0f / L;
-#pragma unroll
-    for (int i = 0; i < DPL; ++i) {
-      const float r = O[i] * inv;
-      out[(s * nh + h) * HD + lane * DPL + i] = r;
-      Os[hh][lane * DPL + i] = r;
-    }
+    attn_merge<HD>(part + (s * nh + h) * nch_grid * PW, nch, lane, out + (s * nh + h) * HD, Os[hh]);
   }
   if (threadIdx.x == 0) st_agent(counters + s * nkv + g, 0u);  // ready for the next call
   if (qt) {
@@ -567,7 +597,7 @@ __device__ __forceinline__ void attn_batch(int64_t bid, const float *__restrict_
 }
 
 template <int HD>
-__global__ void __launch_bounds__(256) k_attn_dec(const float *__restrict__ q, const uint16_t *__restrict__ kc,
+__global__ void __launch_bounds__(256, 3) k_attn_dec(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                   const uint16_t *__restrict__ vc, int64_t s_rows, int nh, int nkv,
                                                   int64_t pos0, const int32_t *__restrict__ pos_dev, int64_t n_ctx,
                                                   int nch_grid, float *part, uint32_t *counters,
@@ -575,11 +605,10 @@ __global__ void __launch_bounds__(256) k_attn_dec(const float *__restrict__ q, c
                                                   float *__restrict__ xd, int32_t *__restrict__ xs) {
   __shared__ uint32_t last;
   __shared__ __attribute__((aligned(16))) float Qs[kMaxGroup][HD];
-  __shared__ __attribute__((aligned(16))) float Os[kMaxGroup][HD];
   __shared__ float Ws[4][kAttnChunk];
   __shared__ AttnKTile<HD> Kt;
   attn_batch<HD>(blockIdx.x, q, kc, vc, s_rows, nh, nkv, pos0, pos_dev, n_ctx, nch_grid, part, counters, out, qt, xq,
-                 xd, xs, Qs, Os, Ws, Kt, last);
+                 xd, xs, Qs, Qs, Ws, Kt, last);
 }
 
 // The same attention for one query row per call (decode), grid nh x nch_grid
@@ -593,7 +622,7 @@ __global__ void __launch_bounds__(256) k_attn_dec(const float *__restrict__ q, c
 // QT 2 also writes the head's Q8 rows (32-blocks) for the projection after it;
 // QT 1 (Q8_K, whose blocks span heads) is not taken.
 template <int HD>
-__global__ void __launch_bounds__(256) k_attn_one(const float *__restrict__ q, const uint16_t *__restrict__ kc,
+__global__ void __launch_bounds__(256, 3) k_attn_one(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                   const uint16_t *__restrict__ vc, int nh, int nkv, int64_t pos0,
                                                   const int32_t *__restrict__ pos_dev, int64_t n_ctx, int nch_grid,
                                                   float *part, uint32_t *counters, float *__restrict__ out, int qt,
@@ -603,18 +632,25 @@ __global__ void __launch_bounds__(256) k_attn_one(const float *__restrict__ q, c
   constexpr int DPL = HD / 64;
   constexpr int PW = HD + 2;  // one chunk partial: m, l, acc[HD]
   __shared__ uint32_t last;
+  // The K tiles hold half of each row per wave (the short path writes and reads
+  // one half after the other), so that three work-groups fit a CU when the
+  // chunks of a long row spread over it.
   __shared__ __attribute__((aligned(16))) float Qs[kMaxGroup][HD];
-  __shared__ __attribute__((aligned(16))) float Os[kMaxGroup][HD];
   __shared__ float Ws[4][kAttnChunk];
   __shared__ __attribute__((aligned(16))) float Lp[kAttnSpanMax][PW];
-  __shared__ AttnKTile<HD> Kt[kAttnSpanMax];
+  union KTiles {
+    uint4 half[kAttnSpanMax][kAttnChunk][KV4 / 2 + 1];
+    AttnKTile<HD> whole;
+  };
+  __shared__ __attribute__((aligned(16))) KTiles Kt;
+  auto &Kh = Kt.half;
   int64_t n = position(pos0, pos_dev) + 1;
   if (n > n_ctx) n = n_ctx;
   const int nch = (int)((n + kAttnChunk - 1) / kAttnChunk);
   if (nch > kAttnSpanMax) {
     if (blockIdx.x < nkv * nch_grid)
       attn_batch<HD>(blockIdx.x, q, kc, vc, 1, nh, nkv, pos0, pos_dev, n_ctx, nch_grid, part, counters, out, qt, xq,
-                     xd, xs, Qs, Os, Ws, Kt[0], last);
+                     xd, xs, Qs, Qs, Ws, Kt.whole, last);
     return;
   }
   if (blockIdx.x >= (unsigned)nh) return;
@@ -627,20 +663,37 @@ __global__ void __launch_bounds__(256) k_attn_one(const float *__restrict__ q, c
   const int64_t p0 = (int64_t)c * kAttnChunk;
   const int np = active ? (int)(n - p0 < kAttnChunk ? n - p0 : kAttnChunk) : 0;
   if (threadIdx.x < HD) Qs[0][threadIdx.x] = q[(int64_t)h * HD + threadIdx.x];
-  uint4 kp[KV4], vp[KV4];
+  typedef uint32_t u4v __attribute__((ext_vector_type(4)));
+  u4v kp[KV4];
+  uint4 vp[KV4];
   if (active) {
 #pragma unroll
-    for (int j = 0; j < KV4; ++j) kp[j] = *(const uint4 *)(kc + attn_piece_off<HD>(kvw, g, p0, np, j, lane));
+    for (int j = 0; j < KV4; ++j) kp[j] = *(const u4v *)(kc + attn_piece_off<HD>(kvw, g, p0, np, j, lane));
 #pragma unroll
     for (int j = 0; j < KV4; ++j) vp[j] = *(const uint4 *)(vc + attn_piece_off<HD>(kvw, g, p0, np, j, lane));
-#pragma unroll
-    for (int j = 0; j < KV4; ++j) Kt[wave].p[j * (64 / KV4) + lane / KV4][lane % KV4] = kp[j];
   }
-  lds_barrier();  // Qs, the K tiles
+  lds_barrier();  // Qs
   if (active) {
+    // K rows through LDS: the first half of every row, then the second
     uint4 kr[KV4];
+    constexpr int HP = KV4 / 2;
+    uint4(*kt)[HP + 1] = Kh[wave];
+    const int r0 = lane / KV4, pc = lane % KV4;
+    if (pc < HP) {
 #pragma unroll
-    for (int j = 0; j < KV4; ++j) kr[j] = Kt[wave].p[lane][j];
+      for (int j = 0; j < KV4; ++j) *(u4v *)&kt[j * (64 / KV4) + r0][pc] = kp[j];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < HP; ++j) kr[j] = kt[lane][j];
+    wave_lds_sync();  // read before the second half overwrites it
+    if (pc >= HP) {
+#pragma unroll
+      for (int j = 0; j < KV4; ++j) *(u4v *)&kt[j * (64 / KV4) + r0][pc - HP] = kp[j];
+    }
+    wave_lds_sync();
+#pragma unroll
+    for (int j = 0; j < HP; ++j) kr[HP + j] = kt[lane][j];
     const float sc_ = attn_score<HD>(Qs[0], kr, lane, np);
     const float m = group_max<64>(sc_);
     const float e = lane < np ? expf(sc_ - m) : 0.0f;
@@ -675,13 +728,13 @@ __global__ void __launch_bounds__(256) k_attn_one(const float *__restrict__ q, c
   for (int i = 0; i < DPL; ++i) {
     const float r = O[i] * inv;
     out[(int64_t)h * HD + lane * DPL + i] = r;
-    Os[0][lane * DPL + i] = r;
+    Qs[0][lane * DPL + i] = r;
   }
   if (qt == 2) {
     wave_lds_sync();  // the head's outputs are in LDS
     const int b = lane >> 3;  // HD / 32 blocks of 8 lanes
     if (b < HD / 32) {
-      const float4 v = *(const float4 *)(&Os[0][0] + 32 * b + 4 * (lane & 7));
+      const float4 v = *(const float4 *)(&Qs[0][0] + 32 * b + 4 * (lane & 7));
       const int64_t blk = (int64_t)h * (HD / 32) + b;
       group8_quant_q8_vals(v, xq + 32 * blk, xd + blk, xs + 2 * blk, lane & 7);
     }
@@ -864,6 +917,10 @@ hipError_t launch_attention(hipStream_t st, const float *q, const uint16_t *kc, 
   if (s_rows <= 0) return hipSuccess;
   if (s_rows == 1) {  // decode
     if (qt == 1) return hipErrorNotSupported;  // a work-group per head writes no Q8_K blocks
+    // A long row at a position the host knows: the batch kernel's work-groups
+    // (a quarter of the LDS) at once.
+    const int64_t n = pos0 + 1 < n_ctx ? pos0 + 1 : n_ctx;
+    if (!pos_dev && n > kAttnSpanMax * kAttnChunk) goto batch;
     const unsigned g1 = (unsigned)((int64_t)nh * supers);
     if (hd == 64)
       KMOE_LAUNCH(k_attn_one<64>, dim3(g1), dim3(256), 0, st, q, kc, vc, nh, nkv, pos0, pos_dev, n_ctx, supers, part,
@@ -875,6 +932,7 @@ hipError_t launch_attention(hipStream_t st, const float *q, const uint16_t *kc, 
       return hipErrorInvalidValue;
     return hipGetLastError();
   }
+batch:
   if (qt == 1 && ((nh / nkv) * hd) % 256 != 0) return hipErrorNotSupported;
   const unsigned grid = (unsigned)((int64_t)nkv * s_rows * supers);
   if (hd == 64)
