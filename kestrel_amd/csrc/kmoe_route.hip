@@ -712,6 +712,128 @@ __global__ void __launch_bounds__(256) k_route_dec(RouteDecArgs a) {
 
 }  // namespace
 
+namespace {
+
+// The same logits for batches: 8 lanes per TQ x TQ tile of (row, token) logits
+// (lane l: chain l of each), 8 row tiles by 4 token tiles per work-group, so
+// that an element read from LDS is used TQ times; one logit per 16 lanes reads
+// two floats per FMA and is bound by that (1777 tokens by 128 rows of 2048:
+// 180-200 us; 4 x 4 tiles 60 us). Columns are staged 256 at a time, chain-major
+// (element 8c + l at l * 36 + c: a lane reads four steps of its chain as 16
+// bytes, eight lanes 128 different bytes of the banks), the next chunk's loads
+// in flight meanwhile. A logit in dot_f32 order keeps the odd steps (its second
+// set of chains) in a second sum; row tiles without one skip that.
+// d % 256 == 0, 16-byte aligned rows, s_rows >= 4, not quant::dot order.
+constexpr int kRtChain = 36;  // a chain's 32 steps of a chunk and 4 words apart
+template <int TQ>
+__global__ void __launch_bounds__(256) k_router_tile(const float *__restrict__ W, int32_t E, int64_t d,
+                                                     const float *__restrict__ X, int64_t S,
+                                                     float *__restrict__ logits, int32_t nlog, int qkind,
+                                                     int8_t *__restrict__ xq, float *__restrict__ xd,
+                                                     int32_t *__restrict__ xs) {
+  constexpr int TE = 8 * TQ, TT = 4 * TQ, NL = (TE + TT) / 4;  // 16-byte loads per thread and chunk
+  __shared__ __attribute__((aligned(16))) float L[TE + TT][8 * kRtChain];
+  if ((int32_t)blockIdx.x >= nlog) {  // the int8 rows of x, as in k_router_logits
+    const int lane = threadIdx.x & 63;
+    const int64_t u = (int64_t)(blockIdx.x - nlog) * 4 + (threadIdx.x >> 6);
+    if (qkind == 1) {
+      if (u < S * (d / 256)) wave_quant_q8k_block(X + u * 256, xq + u * 256, xd + u, xs + u * 16, lane);
+    } else {
+      const int64_t blk = u * 8 + (lane >> 3);
+      if (blk < S * (d / 32)) group8_quant_q8_block(X + blk * 32, xq + blk * 32, xd + blk, xs + blk * 2, lane & 7);
+    }
+    return;
+  }
+  const int tid = threadIdx.x, l = tid & 7, eq = tid >> 3 & 7, tq = tid >> 6;
+  const int nte = (E + TE - 1) / TE;
+  const int e0 = (int)(blockIdx.x % (uint32_t)nte) * TE;
+  const int64_t s0 = (int64_t)(blockIdx.x / (uint32_t)nte) * TT;
+  // dot_f32 order: the rows past the last whole group of 3 of a 48-row tile, the last S % 4 tokens
+  bool dote[TQ], dott[TQ], anydot = false;
+#pragma unroll
+  for (int i = 0; i < TQ; ++i) {
+    const int e = e0 + TQ * eq + i, r0 = e / 48 * 48, tr = E - r0 < 48 ? E - r0 : 48;
+    dote[i] = e - r0 >= tr / 3 * 3;
+    dott[i] = s0 + TQ * tq + i >= S / 4 * 4;
+    anydot = anydot || dote[i] || dott[i];
+  }
+  float4 rv[NL];
+  auto load = [&](int64_t c0) {
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      const int r = 4 * k + (tid >> 6);  // a wave loads one row's 256 columns
+      const float *p;
+      if (r < TE) p = W + (int64_t)(e0 + r < E ? e0 + r : E - 1) * d;
+      else p = X + (s0 + r - TE < S ? s0 + r - TE : S - 1) * d;
+      rv[k] = *(const float4 *)(p + c0 + 4 * (tid & 63));
+    }
+  };
+  float a0[TQ][TQ], a1[TQ][TQ];
+#pragma unroll
+  for (int i = 0; i < TQ; ++i)
+#pragma unroll
+    for (int j = 0; j < TQ; ++j) a0[i][j] = a1[i][j] = 0.0f;
+  load(0);
+  for (int64_t c0 = 0; c0 < d; c0 += 256) {
+    __syncthreads();  // the previous chunk has been read
+#pragma unroll
+    for (int k = 0; k < NL; ++k) {
+      float *p = &L[4 * k + (tid >> 6)][4 * (tid & 1) * kRtChain + (tid & 63) / 2];
+      p[0] = rv[k].x;
+      p[kRtChain] = rv[k].y;
+      p[2 * kRtChain] = rv[k].z;
+      p[3 * kRtChain] = rv[k].w;
+    }
+    __syncthreads();
+    if (c0 + 256 < d) load(c0 + 256);
+    const float *wp = &L[TQ * eq][l * kRtChain], *xp = &L[TE + TQ * tq][l * kRtChain];
+#pragma unroll 2
+    for (int c = 0; c < 32; c += 4) {
+      float w[TQ][4], x[TQ][4];
+#pragma unroll
+      for (int i = 0; i < TQ; ++i) {
+        *(float4 *)w[i] = *(const float4 *)(wp + i * 8 * kRtChain + c);
+        *(float4 *)x[i] = *(const float4 *)(xp + i * 8 * kRtChain + c);
+      }
+      if (!anydot) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < TQ; ++i)
+#pragma unroll
+            for (int j = 0; j < TQ; ++j) a0[i][j] = fmaf(w[i][k], x[j][k], a0[i][j]);
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+#pragma unroll
+          for (int i = 0; i < TQ; ++i)
+#pragma unroll
+            for (int j = 0; j < TQ; ++j) {
+              const bool second = (k & 1) && (dote[i] || dott[j]);
+              const float v = fmaf(w[i][k], x[j][k], second ? a1[i][j] : a0[i][j]);
+              if (second) a1[i][j] = v;
+              else a0[i][j] = v;
+            }
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < TQ; ++i)
+#pragma unroll
+    for (int j = 0; j < TQ; ++j) {
+      float v = a0[i][j];
+      if (dote[i] || dott[j]) v = v + a1[i][j];
+      v = v + __shfl_xor(v, 4);  // hsum
+      v = v + __shfl_xor(v, 2);
+      v = v + __shfl_xor(v, 1);
+      const int e = e0 + TQ * eq + i;
+      const int64_t s = s0 + TQ * tq + j;
+      if (l == 0 && e < E && s < S) logits[s * E + e] = v;
+    }
+}
+
+}  // namespace
+
 hipError_t launch_router_logits(hipStream_t st, const float *router, int32_t n_expert, int64_t d, const float *x,
                                 int64_t s_rows, float *logits, bool qdot, int qkind, int8_t *xq, float *xd,
                                 int32_t *xs) {
@@ -725,6 +847,24 @@ hipError_t launch_router_logits(hipStream_t st, const float *router, int32_t n_e
     KMOE_LAUNCH((k_router_logits<1, 2, 4096>), dim3((unsigned)(blocks + qblocks)), dim3(256), 0, st, router,
                 n_expert, d, x, s_rows, logits, qdot ? 1 : 0, (int32_t)blocks, qkind, xq, xd, xs);
     return hipGetLastError();
+  }
+  // Tiles of 4 x 4 or 2 x 2 logits per 8 lanes, where they still give about a
+  // work-group per CU, or one per two; below that the chains of single logits
+  // run at once on more CUs.
+  if (!qdot && d % 256 == 0 && (((uintptr_t)router | (uintptr_t)x) & 15) == 0) {
+    const int64_t b4 = (s_rows + 15) / 16 * ((n_expert + 31) / 32), b2 = (s_rows + 7) / 8 * ((n_expert + 15) / 16);
+    if (b2 + qblocks <= (int64_t)INT32_MAX && n_expert > 8) {
+      if (b4 >= 200) {
+        KMOE_LAUNCH(k_router_tile<4>, dim3((unsigned)(b4 + qblocks)), dim3(256), 0, st, router, n_expert, d, x, s_rows,
+                    logits, (int32_t)b4, qkind, xq, xd, xs);
+        return hipGetLastError();
+      }
+      if (b2 >= 96) {
+        KMOE_LAUNCH(k_router_tile<2>, dim3((unsigned)(b2 + qblocks)), dim3(256), 0, st, router, n_expert, d, x, s_rows,
+                    logits, (int32_t)b2, qkind, xq, xd, xs);
+        return hipGetLastError();
+      }
+    }
   }
   const int64_t blocks = (s_rows + 3) / 4 * ((n_expert + 3) / 4);
   if (blocks + qblocks > (int64_t)INT32_MAX) return hipErrorInvalidValue;
