@@ -123,6 +123,18 @@ bool f16_plain(int t, int64_t rows, int64_t s_rows) {
 // 947, 96 tokens 963 -> 948; Qwen3 shape 16 tokens 85 -> 109, 96 tokens 248 ->
 // 140, 1777 tokens 2067 -> 702; DeepSeek-V2-Lite shape 32 tokens 255 -> 282,
 // 64 tokens 378 -> 355, 203 tokens 831 -> 356.
+// The int8 regime's expert products. Q6_K and Q8_0 would otherwise run on dot4
+// kernels; Q4_K has int8 matrix-core kernels, which pass over 128 rows of an
+// expert at a time and keep wide parts and few full experts. Layer, us, those
+// -> f16: Mixtral shape with Q6_K down 16 tokens 386 -> 776, 64 tokens 823 ->
+// 784, 512 tokens 5402 -> 1655, Q4_K down 512 tokens 965 -> 1049; DeepSeek-V2-
+// Lite shape (Q8_0 down) 64 tokens 341 -> 346, 128 tokens 413 -> 382; Qwen3
+// shape 128 tokens 186 -> 155, 1777 tokens 1389 -> 509; 32 experts of 1536 by
+// 2048, 400 tokens 169 -> 172, 1777 tokens 523 -> 402.
+bool f16_int(int t, int64_t E, int64_t d, int64_t F, int64_t slots, int64_t max_active) {
+  if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && slots >= (E >= 64 ? 1000 : 3000);
+  return slots >= (t == KMOE_Q6_K ? 16 : 8) * max_active;
+}
 bool f16_experts(int t, int64_t d, int64_t F, int64_t slots) {
   return slots * F >= (t == KMOE_Q6_K ? 600000 : 300000) * (d + F) / d;
 }
@@ -1672,7 +1684,14 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
     const bool more_int = regime == KMOE_REGIME_INT8 || small_rows < 3;
     if (S > small_rows && more_int) {
       hipError_t e = hipErrorNotSupported;
-      if (mfma && gt == KMOE_Q4_K)
+      // the f16 matrix cores (x's piece and sums where y will be) ...
+      if (regime == KMOE_REGIME_INT8 && f16_int(gt, E, d, F, slots, max_active) && (!gd || f16_gemm_i8_captures(gt)))
+        e = timed(c, "moe_gate_up_i8_f16", [&]() {
+          return launch_f16_gemm_i8(st, 0, gt, tier, F, d, rt, (int)E, max_active, S, slots, small_rows + 1, (int)S, w.xq,
+                                    w.xd, w.xs, (uint8_t *)w.y, w.h, gd);
+        });
+      // ... or the int8 ones
+      if (e == hipErrorNotSupported && mfma && gt == KMOE_Q4_K)
         e = timed(c, "moe_gate_up_mfma", [&]() {
           return launch_moe_mfma(st, 0, tier, F, d, rt, regime, max_active, w.xq, w.xd, w.xs, w.h, small_rows + 1,
                                  (int)S, ring_rows, gd);
@@ -1755,7 +1774,13 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
     }
     if (S > small_rows && (regime == KMOE_REGIME_INT8 || small_rows < 3)) {
       hipError_t e = hipErrorNotSupported;
-      if (mfma && dt == KMOE_Q4_K)
+      // (h's piece and sums over its f32 rows, which this regime reads no more)
+      if (regime == KMOE_REGIME_INT8 && f16_int(dt, E, d, F, slots, max_active) && (!dd || f16_gemm_i8_captures(dt)))
+        e = timed(c, "moe_down_i8_f16", [&]() {
+          return launch_f16_gemm_i8(st, 1, dt, tier, d, F, rt, (int)E, max_active, slots, slots, small_rows + 1, (int)S,
+                                    w.hq, w.hd, w.hs, (uint8_t *)w.h, w.y, dd);
+        });
+      if (e == hipErrorNotSupported && mfma && dt == KMOE_Q4_K)
         e = timed(c, "moe_down_mfma", [&]() {
           return launch_moe_mfma(st, 1, tier, d, F, rt, regime, max_active, w.hq, w.hd, w.hs, w.y, small_rows + 1,
                                  (int)S, ring_rows, dd);

@@ -118,6 +118,41 @@ __global__ void __launch_bounds__(64 * WV) k_split_f16(SplitArgs a) {
   }
 }
 
+// ------------------------------------------- int8 activation rows as f16 pieces
+//
+// Rows of int8 values (Q8_K or Q8) as one f16 piece each, exact, in the same
+// order within 8; row r is cols pieces. sums (Q8_K, for Q4_K's minimum term):
+// the sums of 32 from the row's 16-sums, times 2^-5, as above (both pieces
+// together exact: at most 12 bits). One lane per 16 columns.
+__global__ void __launch_bounds__(256) k_i8_f16(const int8_t *__restrict__ q, const int32_t *__restrict__ s16,
+                                                int64_t n16, int64_t cols, uint16_t *__restrict__ planes,
+                                                uint16_t *__restrict__ sums, int64_t sums_stride) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n16) return;
+  const u32x4 v = *(const u32x4 *)(q + 16 * i);
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  u32x4 o[2];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {  // 4 values: (0, 2), (1, 3) of the dword
+    const uint32_t u = w[k] ^ 0x80808080u;
+    const h2 off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    const h2 a = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04020400u)) + off;
+    const h2 b = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, u, 0x04030401u)) + off;
+    o[k >> 1][2 * (k & 1)] = __builtin_bit_cast(uint32_t, a);
+    o[k >> 1][2 * (k & 1) + 1] = __builtin_bit_cast(uint32_t, b);
+  }
+  *(u32x4 *)(planes + 16 * i) = o[0];
+  *(u32x4 *)(planes + 16 * i + 8) = o[1];
+  if (sums && (i & 1) == 0) {
+    const float s = (float)(s16[i] + s16[i + 1]) * 0.03125f;
+    const int64_t r = 16 * i / cols, c = 16 * i - r * cols;
+    _Float16 *p = (_Float16 *)((uint8_t *)sums + r * sums_stride + c / 256 * 32) + (c / 32 % 8);
+    const _Float16 hi = (_Float16)s;
+    p[0] = hi;
+    p[8] = (_Float16)(s - (float)hi);
+  }
+}
+
 // ------------------------------------------------------------------ the product
 
 struct F16Args {
@@ -130,6 +165,8 @@ struct F16Args {
   int n_expert;
   const uint8_t *pw, *pw2;  // plain: GGUF rows; with SwiGLU the gate and the up rows
   int64_t s_rows;           // plain: activation rows
+  const float *ad;          // int8 rows: their block scales [.., cols / 256 or / 32]
+  BlockDbg dbg;             // int8 rows with DBG: per-block integers (gate/down 0, up 1)
 };
 
 __device__ __forceinline__ void lds_dma16(const void *g, uint8_t *lds_wave_base) {
@@ -387,7 +424,13 @@ __device__ __forceinline__ bool find_block(const F16Args &a, int rblocks, int la
 // 278 -> 63. Its MFMAs run a third of the time; the rest is the weights' load
 // requests (32 lines per instruction), the unpacking and the short K loops'
 // ends. Error against 64 bits: 3.1e-7 -> 1.8e-7 (Q4_K matrix).
-template <int T, int MODE, int RT, int NT>
+//
+// INT: int8 activation rows (the int8 path, quant.rs:262-281) as one exact f16
+// piece. A stage's sums are integers below 2^24 for Q4_K (128 * 15*63 * 127)
+// and Q8_0, so they are exact, and join y with the block scales as the int8
+// kernels do; Q6_K's sc * sum is rounded once per 16 columns. DBG adds the
+// exact integers to the capture (Q4_K, Q8_0).
+template <int T, int MODE, int RT, int NT, bool INT = false, bool DBG = false>
 __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   constexpr bool PLAIN = MODE >= 2, TILED = !PLAIN, SWIGLU = MODE == 0 || MODE == 3;
   static_assert(!SWIGLU || RT == 2, "gate and up tiles");
@@ -395,7 +438,9 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   constexpr int G = kGroups<T>, SPG = 8 / G;  // scale groups of a stage, MFMA steps per group
   constexpr int PLANE = BN * 256;             // bytes of one piece plane of a stage
   constexpr int SUMS = T == T_Q4_K ? BN * 32 : 0;  // the superblock's sums, with its second stage
-  __shared__ __attribute__((aligned(16))) uint8_t st0[2 * PLANE], st1[2 * PLANE + SUMS];
+  constexpr int NP = INT ? 1 : 2;                  // pieces per activation
+  constexpr int ADW = T == T_Q8_0 ? 16 : 4, ADS = INT ? BN * ADW : 0;  // block scales of the stage's tokens
+  __shared__ __attribute__((aligned(16))) uint8_t st0[NP * PLANE + ADS], st1[NP * PLANE + ADS + SUMS];
   __shared__ int exs[BN];
   const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -429,23 +474,34 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
     const int64_t p = p0 + tok0 + (t < nbt ? t : nbt - 1);
     return MODE == 0 ? (int64_t)(a.rt.perm[p] / (uint32_t)a.rt.topk) : p;
   };
-  if (tid < BN) exs[tid] = a.x.ex[src_row(tid) * a.x.ex_stride];
+  if constexpr (!INT) {
+    if (tid < BN) exs[tid] = a.x.ex[src_row(tid) * a.x.ex_stride];
+  }
   // direct loads: instruction i of a wave takes tokens 4q .. 4q+3, q = wave * 2 NT + i, of both planes
   uint32_t xsrc[2 * NT];  // (launch: the pieces are below 4 GiB)
 #pragma unroll
   for (int i = 0; i < 2 * NT; ++i) {
     const int t = 4 * (wave * 2 * NT + i) + (lane >> 4);
-    xsrc[i] = (uint32_t)(src_row(t) * 4 * kp) + 16 * ((lane & 15) ^ (t & 15));
+    xsrc[i] = (uint32_t)(src_row(t) * 2 * NP * kp) + 16 * ((lane & 15) ^ (t & 15));
   }
+  const int64_t asrc = INT ? src_row(lane) * (cols / (T == T_Q8_0 ? 32 : 256)) : 0;
   auto load_x = [&](uint8_t *dst, int st) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p)
+    for (int p = 0; p < NP; ++p)
 #pragma unroll
       for (int i = 0; i < 2 * NT; ++i) {
         uint32_t o = xsrc[i];
         asm volatile("" : "+v"(o));  // as in load_raw
         lds_dma16((const uint8_t *)a.x.planes + 2 * kp * p + 256 * (int64_t)st + o, dst + p * PLANE + (wave * 2 * NT + i) * 1024);
       }
+    if constexpr (INT) {  // wave 0: token l's scale of the superblock, or scales of the stage's four blocks
+      if (wave == 0 && lane < BN) {
+        const float *p = a.ad + asrc + (T == T_Q8_0 ? 4 * st : st >> 1);
+        auto *l = (__attribute__((address_space(3))) void *)(dst + NP * PLANE);
+        if constexpr (T == T_Q8_0) __builtin_amdgcn_global_load_lds(p, l, 16, 0, 0);
+        else __builtin_amdgcn_global_load_lds(p, l, 4, 0, 0);
+      }
+    }
   };
   // Q4_K: the superblock's sums of tokens 32w .. 32w+31 by wave w < NT
   uint32_t ssrc = 0;
@@ -454,7 +510,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   // LDS offset of this lane's A piece of K step s: aoff ^ 32s
   const int aoff = 256 * l32 + 16 * (hh ^ (l32 & 15));
 
-  float y[RT][NT][16];
+  float y[RT][NT][16], z[RT][16];  // z: Q6_K with INT
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -466,6 +522,73 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
 #pragma unroll
   for (int i = 0; i < RT; ++i) load_raw<T, TILED>(raw[i], wm[i], wr[i], nb, 0);
 
+  // INT: a group's sums P into y. Lane l's tokens of tile t are 8k + 4(l/32) + 0..3.
+  auto int_epilogue = [&](int t, int gi, f32x16 (&P)[RT], const uint8_t *cur, bool odd, int st,
+                          const float (&g)[RT][G], const h8 (&mo)[RT], const float (&dm)[RT]) {
+    const uint8_t *ads = cur + NP * PLANE;
+    if constexpr (T == T_Q6_K) {  // z += sc * P over the stage, then y += ad * (d * z)
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          z[i][v] = gi == 0 ? g[i][gi] * P[i][v] : fmaf(g[i][gi], P[i][v], z[i][v]);
+          asm volatile("" : "+v"(z[i][v]));
+        }
+      if (gi < G - 1) return;
+    }
+    auto capture = [&](int i, int v, int32_t *const (&arr)[2], float val) {
+      const int tk = 32 * t + 8 * (v >> 2) + 4 * hh + (v & 3);
+      const int64_t r = rbase + (SWIGLU ? 0 : 32 * i) + l32;
+      if (tk < nbt && r < rows)
+        dbg_add(arr[SWIGLU ? i : 0], ((p0 + tok0 + tk) * rows + r) * nb + (T == T_Q8_0 ? 4 * st + gi : st >> 1), (int)val);
+    };
+    // (the minimum term in a pass of its own: its sums live beside P otherwise, and registers run out)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      float sc[4];
+      if constexpr (T == T_Q8_0) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sc[c] = *(const float *)(ads + 16 * (32 * t + 8 * k + 4 * hh + c) + 4 * gi);
+      } else {
+        *(float4 *)sc = *(const float4 *)(ads + 4 * (32 * t + 8 * k + 4 * hh));
+      }
+#pragma unroll
+      for (int i = 0; i < RT; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const int v = 4 * k + c;
+          if constexpr (DBG) capture(i, v, a.dbg.s, P[i][v]);
+          if constexpr (T == T_Q8_0) y[i][t][v] = fmaf(sc[c] * g[i][gi], P[i][v], y[i][t][v]);
+          else if constexpr (T == T_Q6_K) y[i][t][v] = fmaf(sc[c], z[i][v], y[i][t][v]);
+          else y[i][t][v] = fmaf(sc[c], g[i][gi] * P[i][v], y[i][t][v]);
+          asm volatile("" : "+v"(y[i][t][v]));
+        }
+    }
+    if constexpr (T == T_Q4_K) {
+      if (odd) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          const h8 sm = *(const h8 *)(cur + NP * PLANE + ADS + 1024 * t + 32 * l32 + 16 * hh);
+          f32x16 M;
+#pragma unroll
+          for (int v = 0; v < 16; ++v) M[v] = 0.0f;
+          M = __builtin_amdgcn_mfma_f32_32x32x16_f16(sm, mo[i], M, 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            float sc[4];
+            *(float4 *)sc = *(const float4 *)(ads + 4 * (32 * t + 8 * k + 4 * hh));
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+              const int v = 4 * k + c;
+              if constexpr (DBG) capture(i, v, a.dbg.m, M[v]);
+              y[i][t][v] = fmaf(-sc[c], dm[i] * M[v], y[i][t][v]);
+              asm volatile("" : "+v"(y[i][t][v]));
+            }
+          }
+        }
+      }
+    }
+  };
   auto stage = [&](int st, const uint8_t *cur, uint8_t *next, bool odd) {
     __builtin_amdgcn_s_waitcnt(7 << 4);  // this wave's loads of the stage are in, its LDS reads of the last one done
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -477,10 +600,10 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
         uint32_t o = ssrc;
         asm volatile("" : "+v"(o));
         if (!odd && wave < NT)
-          lds_dma16((const uint8_t *)a.x.sums + 32 * (int64_t)(st >> 1) + o, next + 2 * PLANE + wave * 1024);
+          lds_dma16((const uint8_t *)a.x.sums + 32 * (int64_t)(st >> 1) + o, next + NP * PLANE + ADS + wave * 1024);
       }
     }
-    if constexpr (T == T_Q4_K) {  // y -= dmin * sum_j m_j S_j, once per superblock
+    if constexpr (T == T_Q4_K && !INT) {  // y -= dmin * sum_j m_j S_j, once per superblock
       if (odd) {
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
@@ -488,7 +611,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
           const float dm = f16_bits_to_f32(raw[i].hd.x >> 16);
 #pragma unroll
           for (int t = 0; t < NT; ++t) {
-            const h8 sm = *(const h8 *)(cur + 2 * PLANE + 1024 * t + 32 * l32 + 16 * hh);
+            const h8 sm = *(const h8 *)(cur + NP * PLANE + ADS + 1024 * t + 32 * l32 + 16 * hh);
             f32x16 M;
 #pragma unroll
             for (int v = 0; v < 16; ++v) M[v] = 0.0f;
@@ -499,10 +622,16 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
         }
       }
     }
-    h8 w[RT][8];
-    float g[RT][G];
+    h8 w[RT][8], mo[RT];
+    float g[RT][G], dm[RT];
 #pragma unroll
     for (int i = 0; i < RT; ++i) {
+      if constexpr (T == T_Q4_K && INT) {
+        if (odd) {
+          mo[i] = mins_operand(raw[i].hd);
+          dm[i] = f16_bits_to_f32(raw[i].hd.x >> 16);
+        }
+      }
       unpack<T, TILED>(raw[i], st, nb, w[i], g[i]);
 #pragma unroll
       for (int s = 0; s < 8; ++s) asm volatile("" : "+v"(w[i][s]));  // unpacked here, before raw is loaded again
@@ -514,12 +643,21 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       }
     };
     if (T == T_Q4_K || NT == 1) next_weights();
-    // The 16 A pieces of a tile in 4 reads of 4, each issued one read ahead of
-    // its MFMAs. Q4_K: the small pieces of steps 0-3, 4-7, then the large
-    // ones; Q8_0: a block's two steps, small then large; Q6_K: two groups of
-    // one step, small then large.
-    auto pl_of = [](int j, int u) { return T == T_Q4_K ? (j < 2 ? 1 : 0) : T == T_Q8_0 ? (u < 2 ? 1 : 0) : 1 - (u & 1); };
-    auto st_of = [](int j, int u) { return T == T_Q4_K ? 4 * (j & 1) + u : T == T_Q8_0 ? 2 * j + (u & 1) : 2 * j + (u >> 1); };
+    // The A pieces of a tile (16, INT 8) in reads of 4, each issued one read
+    // ahead of its MFMAs. Q4_K: the small pieces of steps 0-3, 4-7, then the
+    // large ones; Q8_0: a block's two steps, small then large; Q6_K: two groups
+    // of one step, small then large; INT: steps 0-3, 4-7.
+    constexpr int NR = INT ? 2 : 4;
+    auto pl_of = [](int j, int u) {
+      return INT ? 0 : T == T_Q4_K ? (j < 2 ? 1 : 0) : T == T_Q8_0 ? (u < 2 ? 1 : 0) : 1 - (u & 1);
+    };
+    auto st_of = [](int j, int u) {
+      return INT ? 4 * j + u : T == T_Q4_K ? 4 * (j & 1) + u : T == T_Q8_0 ? 2 * j + (u & 1) : 2 * j + (u >> 1);
+    };
+    auto first_of = [&](int j, int u) { return INT ? (4 * j + u) % SPG == 0 : (T == T_Q4_K ? j + u : T == T_Q8_0 ? u : u & 1) == 0; };
+    auto last_of = [&](int j, int u) {
+      return INT ? (4 * j + u) % SPG == SPG - 1 : T == T_Q4_K ? j == 3 && u == 3 : T == T_Q8_0 ? u == 3 : (u & 1) == 1;
+    };
     h8 x[2][4];
     auto read = [&](int t, int j) {
 #pragma unroll
@@ -533,14 +671,14 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       if (t >= ntt) break;
       f32x16 P[RT];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if (j < 3) read(t, j + 1);
+      for (int j = 0; j < NR; ++j) {
+        if (j < NR - 1) read(t, j + 1);
         else if (t + 1 < NT) read(t + 1, 0);  // also past the last tile: any LDS bytes
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int s = st_of(j, u), gi = s / SPG;
-          if ((T == T_Q4_K ? j + u : T == T_Q8_0 ? u : u & 1) == 0) {  // a group's first
+          if (first_of(j, u)) {  // a group's first
 #pragma unroll
             for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -548,7 +686,9 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
           }
 #pragma unroll
           for (int i = 0; i < RT; ++i) P[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[j & 1][u], w[i][s], P[i], 0, 0, 0);
-          if (T == T_Q4_K ? j == 3 && u == 3 : T == T_Q8_0 ? u == 3 : (u & 1) == 1) {  // its last
+          if (INT && last_of(j, u)) {
+            int_epilogue(t, gi, P, cur, odd, st, g, mo, dm);
+          } else if (last_of(j, u)) {  // its last
 #pragma unroll
             for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -572,11 +712,11 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
     for (int v = 0; v < 16; ++v) {
       const int tk = 32 * t + 8 * (v >> 2) + 4 * hh + (v & 3);
       if (tk >= nbt) continue;
-      const int sh = -exs[tk];
+      const int sh = INT ? 0 : -exs[tk];
       float *o = a.out + (p0 + tok0 + tk) * rows;
       if constexpr (SWIGLU) {  // g / (1 + exp(-g)) * u
         const int64_t r = rbase + l32;
-        const float gv = ldexpf(y[0][t][v], sh), uv = ldexpf(y[1][t][v], sh);
+        const float gv = INT ? y[0][t][v] : ldexpf(y[0][t][v], sh), uv = INT ? y[1][t][v] : ldexpf(y[1][t][v], sh);
         const float den = 1.0f + expf_cr(-gv);
         const float qv = gv / den;
         if (r < rows) o[r] = qv * uv;
@@ -584,7 +724,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
           const int64_t r = rbase + 32 * i + l32;
-          if (r < rows) o[r] = ldexpf(y[i][t][v], sh);
+          if (r < rows) o[r] = INT ? y[i][t][v] : ldexpf(y[i][t][v], sh);
         }
       }
     }
@@ -630,23 +770,28 @@ int num_cus() {
 }
 
 // blocks: an upper bound of the token blocks over all experts.
-template <int T, int MODE, int RT, int NT>
+template <int T, int MODE, int RT, int NT, bool INT = false, bool DBG = false>
 hipError_t launch_t(hipStream_t st, const F16Args &a, int64_t blocks) {
   constexpr int RPB = MODE == 0 || MODE == 3 ? 128 : 128 * RT;
   const int64_t total = blocks * ((a.rows + RPB - 1) / RPB);
   const unsigned grid = (unsigned)((total + 7) / 8 * 8);
-  KMOE_LAUNCH((k_f16_gemm<T, MODE, RT, NT>), dim3(grid), dim3(256), 0, st, a);
+  KMOE_LAUNCH((k_f16_gemm<T, MODE, RT, NT, INT, DBG>), dim3(grid), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
-template <int T>
+template <int T, bool INT = false, bool DBG = false>
 hipError_t launch_grouped_t(hipStream_t st, int mode, const F16Args &a, int64_t n_slots, int max_active) {
   const int64_t ne = n_slots / a.min_rows < max_active ? n_slots / a.min_rows : max_active;
   if (ne == 0) return hipSuccess;
   const bool wide = n_slots > 32 * (int64_t)max_active;
   const int64_t blocks = n_slots / (wide ? 64 : 32) + ne;
-  if (wide) return mode == 0 ? launch_t<T, 0, 2, 2>(st, a, blocks) : launch_t<T, 1, 2, 2>(st, a, blocks);
-  return mode == 0 ? launch_t<T, 0, 2, 1>(st, a, blocks) : launch_t<T, 1, 2, 1>(st, a, blocks);
+  if constexpr (T == T_Q6_K) {  // a scale per 16 columns: two token tiles need more registers than there are
+    return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne)
+                     : launch_t<T, 1, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne);
+  } else {
+  if (wide) return mode == 0 ? launch_t<T, 0, 2, 2, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 2, INT, DBG>(st, a, blocks);
+  return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 1, INT, DBG>(st, a, blocks);
+  }
 }
 
 template <int T>
@@ -663,7 +808,9 @@ hipError_t launch_plain_t(hipStream_t st, const F16Args &a) {
     }
   }
   const int64_t r2 = (a.rows + 255) / 256;
-  if (r2 * n64 >= 2 * cus) return launch_t<T, 2, 2, 2>(st, a, n64);
+  if constexpr (T != T_Q6_K) {
+    if (r2 * n64 >= 2 * cus) return launch_t<T, 2, 2, 2>(st, a, n64);
+  }
   if (r2 * n32 >= cus) return launch_t<T, 2, 2, 1>(st, a, n32);
   return launch_t<T, 2, 1, 1>(st, a, n32);
 }
@@ -689,6 +836,44 @@ hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier 
     case T_Q4_K: return launch_grouped_t<T_Q4_K>(st, mode, a, n_slots, max_active);
     case T_Q6_K: return launch_grouped_t<T_Q6_K>(st, mode, a, n_slots, max_active);
     default: return launch_grouped_t<T_Q8_0>(st, mode, a, n_slots, max_active);
+  }
+}
+
+bool f16_gemm_i8_captures(int type) { return type == T_Q4_K || type == T_Q8_0; }
+
+hipError_t launch_f16_gemm_i8(hipStream_t st, int mode, int type, const ExpertTier &tier, int64_t rows, int64_t cols,
+                              const Routing &rt, int n_expert, int max_active, int64_t n_rows, int64_t n_slots,
+                              int min_rows, int max_rows, const int8_t *q, const float *ad, const int32_t *s16,
+                              uint8_t *scratch, float *out, const BlockDbg *dbg) {
+  if (!f16_gemm_supported(type, rows, cols, n_slots) || cols % 128 || min_rows < 1 || ((uintptr_t)q & 15u) ||
+      ((uintptr_t)ad & 15u) || ((uintptr_t)scratch & 15u) || (dbg && !f16_gemm_i8_captures(type)))
+    return hipErrorNotSupported;
+  if (max_active <= 0 || max_rows < min_rows) return hipSuccess;
+  const int64_t n16 = n_rows * (cols / 16);
+  F16Args a{};
+  a.x.planes = (uint16_t *)scratch;
+  a.x.sums = type == T_Q4_K ? (uint16_t *)(scratch + 2 * n_rows * cols) : nullptr;
+  a.x.sums_stride = cols / 8;
+  hipLaunchKernelGGL(k_i8_f16, dim3((unsigned)((n16 + 255) / 256)), dim3(256), 0, st, q, s16, n16, cols, a.x.planes,
+                     a.x.sums, a.x.sums_stride);
+  a.tier = tier;
+  a.rt = rt;
+  a.rows = rows;
+  a.cols = cols;
+  a.out = out;
+  a.min_rows = min_rows;
+  a.max_rows = max_rows;
+  a.n_expert = n_expert;
+  a.ad = ad;
+  if (dbg) {
+    a.dbg = *dbg;
+    return type == T_Q4_K ? launch_grouped_t<T_Q4_K, true, true>(st, mode, a, n_slots, max_active)
+                          : launch_grouped_t<T_Q8_0, true, true>(st, mode, a, n_slots, max_active);
+  }
+  switch (type) {
+    case T_Q4_K: return launch_grouped_t<T_Q4_K, true>(st, mode, a, n_slots, max_active);
+    case T_Q6_K: return launch_grouped_t<T_Q6_K, true>(st, mode, a, n_slots, max_active);
+    default: return launch_grouped_t<T_Q8_0, true>(st, mode, a, n_slots, max_active);
   }
 }
 

@@ -138,3 +138,50 @@ def test_a_budget_without_room_for_the_pieces_keeps_the_other_kernels():
     assert c.profile_read("f16_gemm")[1] == 0 and c.profile_read("f32_rows_plain")[1] == 1
     c.close()
     assert rel_l2(full, tight) < 2e-6
+
+
+# the int8 regime's ragged experts: every weight type, the per-block integers
+# of the kernels that ran (Q4_K, Q8_0), with blocks and activations at their
+# extremes so that a stage's sums reach their largest
+@pytest.mark.parametrize("E,k,d,F,S,gt,dt", [(70, 3, 256, 384, 401, Q4_K, Q8_0), (66, 2, 512, 256, 700, Q4_K, Q4_K),
+                                             (5, 2, 256, 512, 90, Q6_K, Q6_K), (6, 1, 384, 256, 130, Q8_0, Q6_K)])
+def test_int8_regime_expert_layers(ctx, E, k, d, F, S, gt, dt):
+    import torch
+    from oracle import pyoracle as orc
+
+    spec = LayerSpec(E, k, d, F, gt, seed=E + S, down_type=dt, zipf=1.2)
+    if gt == Q4_K:  # all-ones scales, minimums and nibbles
+        for e in range(E):
+            spec.up[e].reshape(-1, 144)[::2, 4:] = 0xFF
+    x = orc.normal(S, S * d).reshape(S, d) + np.float32(1.0)
+    x[::3] = np.sign(x[::3]) * 3.0
+    spec.upload(ctx, S)
+    xd = torch.from_numpy(x).cuda()
+    ctx.set_regime(1)
+    try:
+        n0 = [ctx.profile_read(n)[1] for n in ("moe_gate_up_i8_f16", "moe_down_i8_f16")]
+        out = ctx.moe_ffn(S, xd).cpu().numpy()
+        assert [ctx.profile_read(n)[1] for n in ("moe_gate_up_i8_f16", "moe_down_i8_f16")] == [n + 1 for n in n0]
+        cap_out, cap = ctx.moe_ffn_dbg(S, xd, k, F, gt, dt)
+        idx, _, perm, off = (t.cpu().numpy() for t in ctx.last_routing(S, k, E))
+    finally:
+        ctx.set_regime(0)
+    layer = spec.oracle_layer()
+    assert np.array_equal(idx.astype(np.uint32), layer.route(x)[0])
+    assert rel_l2(out, layer.moe_ffn(x, 1)) < 1e-3
+    if Q6_K not in (gt, dt):
+        assert np.array_equal(out.view(np.uint32), cap_out.cpu().numpy().view(np.uint32))
+    if gt != Q4_K:
+        return
+    cap = {n: v.cpu().numpy() for n, v in cap.items()}
+    off = off.view(np.uint32)
+    q, _, bs = orc.q8k_quantize(x)
+    big = int(np.argmax(np.diff(off.astype(np.int64))))
+    for e in (big, int(np.argmin(np.where(np.diff(off.astype(np.int64)) > 4, np.diff(off.astype(np.int64)), 1 << 30)))):
+        for p in (int(off[e]), int(off[e + 1]) - 1):
+            tok = int(perm.view(np.uint32)[p]) // k
+            for r in (0, F // 2 + 1, F - 1):
+                row = spec.up[e].reshape(F, -1)[r]
+                s, m = orc.q4k_block_acc(row, d, q.reshape(S, d)[tok], bs.reshape(S, -1)[tok])
+                assert np.array_equal(cap["up_sumi"].reshape(S * k, F, -1)[p, r], s)
+                assert np.array_equal(cap["up_mins"].reshape(S * k, F, -1)[p, r], m)
