@@ -107,22 +107,20 @@ static std::mutex g_scratch_mu;
 // Device completion counters per context (words used by the decode router).
 constexpr int kCounterWords = 64;
 constexpr int kNormDone = 1;  // the decode router's residual writer (kmoe_norm_moe_ffn)
-// Where the f32 regime takes the f16 matrix cores (kmoe_f16gemm.hip). A
-// work-group there walks all columns in stages of one memory round trip each,
-// so a product that does not fill the chip costs that chain whatever its
-// size, while the kernels for few rows shrink with it. Measured (us, those ->
-// f16), one matrix: Q4_K 4096x4096 64 rows 28 -> 39, 96 rows 42 -> 40, 512
-// rows 184 -> 74; 2048x2816 128 rows 21 -> 26, 256 rows 50 -> 28; Q6_K
-// 4096x4096 16 rows 49 -> 66, 24 rows 70 -> 66, 128 rows 312 -> 69; Q8_0
-// 2048x2816 24 rows 40 -> 43, 48 rows 68 -> 43.
-bool f16_plain(int t, int64_t rows, int64_t s_rows) {
-  return t == KMOE_Q4_K ? s_rows >= 24 && s_rows * rows >= 390000 : s_rows >= 4 && s_rows * rows >= 90000;
+// Where the f32 regime takes the f16 matrix cores (kmoe_f16gemm.hip): below a
+// few rows' worth of work the weights' walk through its stages costs more than
+// the kernels for few rows. Measured (us, those -> f16), one matrix: Q4_K
+// 2048x2816 64 rows 15.6 -> 17.2, 96 rows 20.8 -> 18.1, 3072x2048 64 rows 16.0
+// -> 18.1, 4096x4096 32 rows 19.9 -> 18.6, 512 rows 184 -> 68; Q6_K 2048x2816
+// 8 rows 22.0 -> 23.5, 4096x4096 8 rows 33.6 -> 23.4, 128 rows 312 -> 34; Q8_0
+// 3072x2048 16 rows 22.5 -> 25.7, 24 rows 32.6 -> 25.9.
+bool f16_plain(int t, int64_t rows, int64_t cols, int64_t s_rows) {
+  const double work = (double)s_rows * rows * cols;
+  // (many outputs of short rows: no chain to wait for, the stages' loads cost the same)
+  const int64_t outs = s_rows * rows;
+  return t == KMOE_Q4_K ? s_rows >= 24 && (work >= 500e6 || outs >= 390000)
+                        : s_rows >= 4 && (work >= 130e6 || outs >= 90000);
 }
-// Expert layers (whole layer, us): Mixtral shape 48 tokens 411 -> 595, 64
-// tokens 656 -> 600, 512 tokens 3596 -> 1195; with Q6_K down 64 tokens 798 ->
-// 947, 96 tokens 963 -> 948; Qwen3 shape 16 tokens 85 -> 109, 96 tokens 248 ->
-// 140, 1777 tokens 2067 -> 702; DeepSeek-V2-Lite shape 32 tokens 255 -> 282,
-// 64 tokens 378 -> 355, 203 tokens 831 -> 356.
 // The int8 regime's expert products. Q6_K and Q8_0 would otherwise run on dot4
 // kernels; Q4_K has int8 matrix-core kernels, which pass over 128 rows of an
 // expert at a time and keep wide parts and few full experts. Layer, us, those
@@ -135,8 +133,21 @@ bool f16_int(int t, int64_t E, int64_t d, int64_t F, int64_t slots, int64_t max_
   if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && slots >= (E >= 64 ? 1000 : 3000);
   return slots >= (t == KMOE_Q6_K ? 16 : 8) * max_active;
 }
+// Expert layers, gate/up (whole layer, us): Mixtral shape 48 tokens 411 -> 488,
+// 64 tokens 656 -> 488 (both with the down product as below); Qwen3 shape 16
+// tokens 85 -> 109, 96 tokens 248 -> 140; 32 experts of 1536 by 2048, 64 tokens
+// 145 -> 130; DeepSeek-V2-Lite shape 32 tokens 255 -> 282, 64 tokens 378 -> 355.
 bool f16_experts(int t, int64_t d, int64_t F, int64_t slots) {
-  return slots * F >= (t == KMOE_Q6_K ? 600000 : 300000) * (d + F) / d;
+  const int64_t lo = t == KMOE_Q6_K ? 600000 : d * F <= (int64_t)8 << 20 ? 300000 : 400000;
+  return slots * F >= lo * (d + F) / d;
+}
+// Down (its columns split where the grid is small): Q4_K Mixtral shape 4 tokens
+// 142 -> 146, 8 tokens 283 -> 268, 24 tokens 515 -> 475; 2048 by 1536, 16 tokens
+// 94 -> 103; Q6_K Mixtral shape 16 tokens 527 -> 562, 24 tokens 614 -> 605, 64
+// tokens 808 -> 643; Q8_0 2048 by 1408, 32 tokens 231 -> 234, 64 tokens 360 -> 336.
+bool f16_down(int t, int64_t d, int64_t F, int64_t slots, int64_t max_active) {
+  return slots >= 32 * max_active ||
+         (double)slots * d * F >= (t == KMOE_Q4_K ? 0.9e9 : t == KMOE_Q6_K ? 2.5e9 : 1.0e9);
 }
 constexpr int kFewRows = 3;   // decode batches over narrow rows: experts of 1..3 rows take launch_few_int
 
@@ -529,6 +540,8 @@ struct QRows {
   float *part;
   int64_t part_floats;
   F16Rows xf;  // the f32 regime's activation pieces, over the same bytes (planes null: no room for them)
+  float *xf_part = nullptr;  // and the partial sums of their products
+  int64_t xf_part_floats = 0;
 };
 QRows carve_qrows(uint8_t *base, int64_t s_rows, int64_t cols, size_t *total, int64_t part_floats = 0) {
   Carver cv{base};
@@ -560,7 +573,13 @@ F16Rows carve_f16(uint8_t *base, int64_t s_rows, int64_t cols, size_t *total) {
 // push the workspace past the VRAM budget, or grow it inside a graph capture.
 int matmul_ws(kmoe_ctx *c, int t, int64_t rows, int64_t s_rows, int64_t cols, int64_t part_floats, size_t need, QRows *qr) {
   size_t f16 = 0;
-  if (f16_plain(t, rows, s_rows) && f16_gemm_supported(t, rows, cols, s_rows)) carve_f16(nullptr, s_rows, cols, &f16);
+  int64_t pf = 0;
+  size_t pieces = 0;
+  if (f16_plain(t, rows, cols, s_rows) && f16_gemm_supported(t, rows, cols, s_rows)) {
+    pf = f16_gemm_part_floats(t, rows, cols, s_rows);
+    carve_f16(nullptr, s_rows, cols, &pieces);
+    f16 = pieces + align_up((size_t)pf * 4);
+  }
   size_t want = f16 > need ? f16 : need;
   if (want > need && want > c->ws_size) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
@@ -574,7 +593,11 @@ int matmul_ws(kmoe_ctx *c, int t, int64_t rows, int64_t s_rows, int64_t cols, in
   if (rc) return rc;
   size_t n = 0;
   *qr = carve_qrows(c->ws, s_rows, cols, &n, part_floats);
-  if (f16 && f16 <= c->ws_size) qr->xf = carve_f16(c->ws, s_rows, cols, &n);
+  if (f16 && f16 <= c->ws_size) {
+    qr->xf = carve_f16(c->ws, s_rows, cols, &n);
+    qr->xf_part = (float *)(c->ws + pieces);
+    qr->xf_part_floats = pf;
+  }
   return KMOE_OK;
 }
 
@@ -617,7 +640,8 @@ int matmul_core(kmoe_ctx *c, int t, const uint8_t *w, int64_t rows, int64_t cols
       hipError_t e = timed(c, "split_f16", [&]() { return launch_split_f16(c->stream, x, s_rows, cols, xf); });
       if (e == hipSuccess)
         e = timed(c, "f16_gemm", [&]() {
-          return launch_f16_gemm_plain(c->stream, t, w, rows, cols, xf, s_rows, out);
+          return launch_f16_gemm_plain(c->stream, t, w, rows, cols, xf, s_rows, out, nullptr, qr.xf_part,
+                                       qr.xf_part_floats);
         });
       if (e == hipSuccess) return KMOE_OK;
       if (e != hipErrorNotSupported) HIP_OK(c, e);
@@ -1795,7 +1819,7 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
     int f32_done = 0;
     // h's pieces in place; their sums and exponents in the slots' int8 sums and
     // scales, which the f32 regime's slots do not use
-    if (f16_experts(dt, d, F, slots) && f16_gemm_supported(dt, d, F, slots) && F % 128 == 0) {
+    if (f16_down(dt, d, F, slots, max_active) && f16_gemm_supported(dt, d, F, slots) && F % 128 == 0) {
       F16Rows hf;
       hf.planes = (uint16_t *)w.h;
       hf.sums = dt == KMOE_Q4_K ? (uint16_t *)w.hs : nullptr;
@@ -1807,7 +1831,8 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
       });
       if (e == hipSuccess) {  // from here on these slots' h is pieces only
         LAUNCH(c, "moe_down_f16",
-               launch_f16_gemm(st, 1, dt, tier, d, F, rt, (int)E, max_active, slots, f32_lo, f32_hi, hf, w.y));
+               launch_f16_gemm(st, 1, dt, tier, d, F, rt, (int)E, max_active, slots, f32_lo, f32_hi, hf, w.y, w.part,
+                               w.part_floats, w.idx));
         f32_done = f32_hi;
       } else if (e != hipErrorNotSupported) {
         HIP_OK(c, e);
@@ -1888,7 +1913,7 @@ done:
       LAUNCH(c, "shared_swiglu", launch_swiglu(st, gs, us, S * Fs));
     }
     bool ys_done = false;
-    if (!int_path(regime, S) && f16_plain(t2, d, S) && f16_gemm_supported(t2, d, Fs, S) && Fs % 128 == 0) {
+    if (!int_path(regime, S) && f16_plain(t2, d, Fs, S) && f16_gemm_supported(t2, d, Fs, S) && Fs % 128 == 0) {
       // the SwiGLU rows' pieces in place, their sums and exponents in the int8 scratch
       F16Rows gf;
       gf.planes = (uint16_t *)gs;
@@ -1900,7 +1925,8 @@ done:
       if (((uintptr_t)(SH.arena + SH.off[2]) & al) == 0)
         e = timed(c, "split_f16", [&]() { return launch_split_f16(st, gs, S, Fs, gf); });
       if (e == hipSuccess) {
-        LAUNCH(c, "shared_down_f16", launch_f16_gemm_plain(st, t2, SH.arena + SH.off[2], d, Fs, gf, S, ys));
+        LAUNCH(c, "shared_down_f16", launch_f16_gemm_plain(st, t2, SH.arena + SH.off[2], d, Fs, gf, S, ys, nullptr,
+                                                                  qr.part, qr.part_floats));
         ys_done = true;
       } else if (e != hipErrorNotSupported) {
         HIP_OK(c, e);

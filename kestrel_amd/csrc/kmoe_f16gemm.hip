@@ -165,6 +165,8 @@ struct F16Args {
   int n_expert;
   const uint8_t *pw, *pw2;  // plain: GGUF rows; with SwiGLU the gate and the up rows
   int64_t s_rows;           // plain: activation rows
+  int split_stages;         // columns split over blockIdx.y: stages per split (even; 0: no split), each split's
+  int64_t split_stride;     // sums at out + split * split_stride
   const float *ad;          // int8 rows: their block scales [.., cols / 256 or / 32]
   BlockDbg dbg;             // int8 rows with DBG: per-block integers (gate/down 0, up 1)
 };
@@ -458,7 +460,9 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   const int64_t nb = cols / (T == T_Q8_0 ? 32 : 256);
   const int64_t row_bytes = nb * (T == T_Q4_K ? 144 : T == T_Q6_K ? 210 : 34);
   const int64_t kp = (cols + 127) / 128 * 128;
-  const int nst = (int)(kp / 128);
+  const int nst_all = (int)(kp / 128);
+  const int st_lo = a.split_stages ? (int)blockIdx.y * a.split_stages : 0;
+  const int nst = a.split_stages && st_lo + a.split_stages < nst_all ? st_lo + a.split_stages : nst_all;
   const int64_t rbase = (int64_t)rb * RPB + wave * (SWIGLU ? 32 : 32 * RT);
   const uint8_t *wm[RT];  // matrix (uniform) and row offset of each tile (launch: a matrix is below 4 GiB)
   uint32_t wr[RT];
@@ -518,9 +522,9 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
 #pragma unroll
       for (int v = 0; v < 16; ++v) y[i][t][v] = 0.0f;
   Raw<T> raw[RT];
-  load_x(st0, 0);
+  load_x(st0, st_lo);
 #pragma unroll
-  for (int i = 0; i < RT; ++i) load_raw<T, TILED>(raw[i], wm[i], wr[i], nb, 0);
+  for (int i = 0; i < RT; ++i) load_raw<T, TILED>(raw[i], wm[i], wr[i], nb, st_lo);
 
   // INT: a group's sums P into y. Lane l's tokens of tile t are 8k + 4(l/32) + 0..3.
   auto int_epilogue = [&](int t, int gi, f32x16 (&P)[RT], const uint8_t *cur, bool odd, int st,
@@ -702,7 +706,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       }
     }
   };
-  for (int st = 0; st < nst; st += 2) {
+  for (int st = st_lo; st < nst; st += 2) {
     stage(st, st0, st1, false);
     if (st + 1 < nst) stage(st + 1, st1, st0, true);
   }
@@ -713,7 +717,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       const int tk = 32 * t + 8 * (v >> 2) + 4 * hh + (v & 3);
       if (tk >= nbt) continue;
       const int sh = INT ? 0 : -exs[tk];
-      float *o = a.out + (p0 + tok0 + tk) * rows;
+      float *o = a.out + (p0 + tok0 + tk) * rows + (SWIGLU ? 0 : (int64_t)blockIdx.y * a.split_stride);
       if constexpr (SWIGLU) {  // g / (1 + exp(-g)) * u
         const int64_t r = rbase + l32;
         const float gv = INT ? y[0][t][v] : ldexpf(y[0][t][v], sh), uv = INT ? y[1][t][v] : ldexpf(y[1][t][v], sh);
@@ -729,6 +733,29 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       }
     }
   }
+}
+
+// out[p] = the column splits' sums of row p, in split order. idx (grouped rows):
+// only rows of experts with at least min_rows rows.
+__global__ void __launch_bounds__(256) k_split_sum(const float *__restrict__ part, int ks, int64_t stride, int64_t rows,
+                                                   int64_t n4, float *__restrict__ out,
+                                                   const uint32_t *__restrict__ idx, const uint32_t *__restrict__ perm,
+                                                   const uint32_t *__restrict__ offsets, int min_rows) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n4) return;
+  if (idx) {
+    const uint32_t e = idx[perm[4 * i / rows]];
+    if ((int)(offsets[e + 1] - offsets[e]) < min_rows) return;
+  }
+  float4 s = *(const float4 *)(part + 4 * i);
+  for (int k = 1; k < ks; ++k) {
+    const float4 v = *(const float4 *)(part + k * stride + 4 * i);
+    s.x += v.x;
+    s.y += v.y;
+    s.z += v.z;
+    s.w += v.w;
+  }
+  *(float4 *)(out + 4 * i) = s;
 }
 
 constexpr int64_t kSplitCols = 16384;  // the widest row k_split_f16 takes
@@ -769,33 +796,84 @@ int num_cus() {
   return cus;
 }
 
+int64_t splits_for(int64_t total, int nst, int rt) {
+  const int64_t ks = (rt == 1 ? 4 : 2) * (int64_t)num_cus() / (total > 0 ? total : 1);
+  return ks < nst / 6 ? ks : nst / 6;
+}
+
+// Where the partial sums of a column split may go; grouped: all slots and their flat expert choice.
+struct Split {
+  float *part = nullptr;
+  int64_t part_floats = 0, n_slots = 0;
+  const uint32_t *idx = nullptr;
+};
+
 // blocks: an upper bound of the token blocks over all experts.
 template <int T, int MODE, int RT, int NT, bool INT = false, bool DBG = false>
-hipError_t launch_t(hipStream_t st, const F16Args &a, int64_t blocks) {
+hipError_t launch_t(hipStream_t st, const F16Args &a, int64_t blocks, const Split &sp = {}) {
   constexpr int RPB = MODE == 0 || MODE == 3 ? 128 : 128 * RT;
   const int64_t total = blocks * ((a.rows + RPB - 1) / RPB);
   const unsigned grid = (unsigned)((total + 7) / 8 * 8);
+  if constexpr (!INT && (MODE == 1 || MODE == 2)) {
+    // A grid that leaves the chip idle splits the columns, at least six stages
+    // (768 columns) to a work-group, over as many as fill it twice (one row
+    // tile per wave: four times) and the partial sums' buffer holds. 4096x4096
+    // by 16 rows: Q4_K 37 -> 17.5 us, Q6_K 66 -> 24, Q8_0 75 -> 26.
+    const int nst = (int)((a.cols + 127) / 128);
+    const int64_t stride = (MODE == 1 ? sp.n_slots : a.s_rows) * a.rows;
+    int64_t ks = splits_for(total, nst, RT);
+    if (ks * stride > sp.part_floats) ks = sp.part_floats / stride;
+    if (ks >= 2 && a.rows % 4 == 0 && stride / 4 < (int64_t)INT32_MAX * 128) {
+      F16Args b = a;
+      b.split_stages = (int)((nst + ks - 1) / ks + 1) / 2 * 2;
+      b.split_stride = stride;
+      b.out = sp.part;
+      ks = (nst + b.split_stages - 1) / b.split_stages;
+      KMOE_LAUNCH((k_f16_gemm<T, MODE, RT, NT, INT, DBG>), dim3(grid, (unsigned)ks), dim3(256), 0, st, b);
+      hipLaunchKernelGGL(k_split_sum, dim3((unsigned)((stride / 4 + 255) / 256)), dim3(256), 0, st, sp.part, (int)ks,
+                         stride, a.rows, stride / 4, a.out, MODE == 1 ? sp.idx : nullptr, a.rt.perm, a.rt.offsets,
+                         a.min_rows);
+      return hipGetLastError();
+    }
+  }
   KMOE_LAUNCH((k_f16_gemm<T, MODE, RT, NT, INT, DBG>), dim3(grid), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
 template <int T, bool INT = false, bool DBG = false>
-hipError_t launch_grouped_t(hipStream_t st, int mode, const F16Args &a, int64_t n_slots, int max_active) {
+hipError_t launch_grouped_t(hipStream_t st, int mode, const F16Args &a, int64_t n_slots, int max_active,
+                            const Split &sp = {}) {
   const int64_t ne = n_slots / a.min_rows < max_active ? n_slots / a.min_rows : max_active;
   if (ne == 0) return hipSuccess;
+  if constexpr (!INT) {  // few token blocks: one row tile per wave, columns split
+    if (mode == 1 && (n_slots / 32 + ne) * ((a.rows + 255) / 256) < 2 * num_cus())
+      return launch_t<T, 1, 1, 1>(st, a, n_slots / 32 + ne, sp);
+  }
   const bool wide = n_slots > 32 * (int64_t)max_active;
   const int64_t blocks = n_slots / (wide ? 64 : 32) + ne;
   if constexpr (T == T_Q6_K) {  // a scale per 16 columns: two token tiles need more registers than there are
     return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne)
-                     : launch_t<T, 1, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne);
+                     : launch_t<T, 1, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne, sp);
   } else {
-  if (wide) return mode == 0 ? launch_t<T, 0, 2, 2, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 2, INT, DBG>(st, a, blocks);
-  return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 1, INT, DBG>(st, a, blocks);
+  if (wide) return mode == 0 ? launch_t<T, 0, 2, 2, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 2, INT, DBG>(st, a, blocks, sp);
+  return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 1, INT, DBG>(st, a, blocks, sp);
   }
 }
 
+// Row tiles per wave, token tiles and token blocks of a plain product: the
+// largest tile that still fills the chip (twice, where two tiles of tokens do).
+struct PlainShape {
+  int rt, nt;
+  int64_t blocks;
+};
+PlainShape plain_shape(int type, int64_t rows, int64_t s_rows) {
+  const int64_t cus = num_cus(), r2 = (rows + 255) / 256, n64 = (s_rows + 63) / 64, n32 = (s_rows + 31) / 32;
+  if (type != T_Q6_K && r2 * n64 >= 2 * cus) return {2, 2, n64};
+  return {r2 * n32 >= cus ? 2 : 1, 1, n32};
+}
+
 template <int T>
-hipError_t launch_plain_t(hipStream_t st, const F16Args &a) {
+hipError_t launch_plain_t(hipStream_t st, const F16Args &a, const Split &sp) {
   const int64_t cus = num_cus();
   const int64_t n64 = (a.s_rows + 63) / 64, n32 = (a.s_rows + 31) / 32;
   if (a.pw2) {
@@ -807,19 +885,27 @@ hipError_t launch_plain_t(hipStream_t st, const F16Args &a) {
       return hipErrorNotSupported;
     }
   }
-  const int64_t r2 = (a.rows + 255) / 256;
+  const PlainShape p = plain_shape(T, a.rows, a.s_rows);
   if constexpr (T != T_Q6_K) {
-    if (r2 * n64 >= 2 * cus) return launch_t<T, 2, 2, 2>(st, a, n64);
+    if (p.nt == 2) return launch_t<T, 2, 2, 2>(st, a, p.blocks, sp);
   }
-  if (r2 * n32 >= cus) return launch_t<T, 2, 2, 1>(st, a, n32);
-  return launch_t<T, 2, 1, 1>(st, a, n32);
+  if (p.rt == 2) return launch_t<T, 2, 2, 1>(st, a, p.blocks, sp);
+  return launch_t<T, 2, 1, 1>(st, a, p.blocks, sp);
 }
 
 }  // namespace
 
+int64_t f16_gemm_part_floats(int type, int64_t rows, int64_t cols, int64_t s_rows) {
+  const PlainShape p = plain_shape(type, rows, s_rows);
+  const int64_t ks = splits_for(p.blocks * ((rows + 128 * p.rt - 1) / (128 * p.rt)), (int)((cols + 127) / 128), p.rt);
+  return ks > 1 && rows % 4 == 0 ? ks * s_rows * rows : 0;
+}
+
 hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier &tier, int64_t rows, int64_t cols,
                            const Routing &rt, int n_expert, int max_active, int64_t n_slots, int min_rows,
-                           int max_rows, const F16Rows &x, float *out) {
+                           int max_rows, const F16Rows &x, float *out, float *part, int64_t part_floats,
+                           const uint32_t *idx) {
+  const Split sp{part, idx ? part_floats : 0, n_slots, idx};
   if (!f16_gemm_supported(type, rows, cols, n_slots) || min_rows < 1) return hipErrorNotSupported;
   if (max_active <= 0 || max_rows < min_rows) return hipSuccess;
   F16Args a{};
@@ -833,9 +919,9 @@ hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier 
   a.max_rows = max_rows;
   a.n_expert = n_expert;
   switch (type) {
-    case T_Q4_K: return launch_grouped_t<T_Q4_K>(st, mode, a, n_slots, max_active);
-    case T_Q6_K: return launch_grouped_t<T_Q6_K>(st, mode, a, n_slots, max_active);
-    default: return launch_grouped_t<T_Q8_0>(st, mode, a, n_slots, max_active);
+    case T_Q4_K: return launch_grouped_t<T_Q4_K>(st, mode, a, n_slots, max_active, sp);
+    case T_Q6_K: return launch_grouped_t<T_Q6_K>(st, mode, a, n_slots, max_active, sp);
+    default: return launch_grouped_t<T_Q8_0>(st, mode, a, n_slots, max_active, sp);
   }
 }
 
@@ -878,7 +964,9 @@ hipError_t launch_f16_gemm_i8(hipStream_t st, int mode, int type, const ExpertTi
 }
 
 hipError_t launch_f16_gemm_plain(hipStream_t st, int type, const uint8_t *w, int64_t rows, int64_t cols,
-                                 const F16Rows &x, int64_t s_rows, float *out, const uint8_t *w_up) {
+                                 const F16Rows &x, int64_t s_rows, float *out, const uint8_t *w_up, float *part,
+                                 int64_t part_floats) {
+  const Split sp{part, part_floats, s_rows, nullptr};
   const uintptr_t al = type == T_Q4_K ? 15u : 1u;
   if (!f16_gemm_supported(type, rows, cols, s_rows) || ((uintptr_t)w & al) || ((uintptr_t)w_up & al))
     return hipErrorNotSupported;
@@ -891,9 +979,9 @@ hipError_t launch_f16_gemm_plain(hipStream_t st, int type, const uint8_t *w, int
   a.pw2 = w_up;
   a.s_rows = s_rows;
   switch (type) {
-    case T_Q4_K: return launch_plain_t<T_Q4_K>(st, a);
-    case T_Q6_K: return launch_plain_t<T_Q6_K>(st, a);
-    default: return launch_plain_t<T_Q8_0>(st, a);
+    case T_Q4_K: return launch_plain_t<T_Q4_K>(st, a, sp);
+    case T_Q6_K: return launch_plain_t<T_Q6_K>(st, a, sp);
+    default: return launch_plain_t<T_Q8_0>(st, a, sp);
   }
 }
 

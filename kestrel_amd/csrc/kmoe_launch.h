@@ -282,12 +282,16 @@ bool f16_gemm_supported(int type, int64_t rows, int64_t cols, int64_t n);
 // of experts with at least min_rows rows are converted.
 hipError_t launch_split_f16(hipStream_t st, const float *x, int64_t rows, int64_t cols, const F16Rows &o,
                             const Routing *rt = nullptr, const uint32_t *idx = nullptr, int min_rows = 0);
+// part (16-byte aligned): partial sums where a small grid splits the columns
+// (products without SwiGLU); grouped also needs idx.
+int64_t f16_gemm_part_floats(int type, int64_t rows, int64_t cols, int64_t s_rows);  // what a plain product uses of it
 // Grouped, experts with min_rows..max_rows rows: mode 0 gate/up + SwiGLU (x:
 // the tokens' rows) into out [slots, rows], mode 1 down (x: the slots' rows).
 // hipErrorNotSupported (nothing launched) for other types or shapes.
 hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier &tier, int64_t rows, int64_t cols,
                            const Routing &rt, int n_expert, int max_active, int64_t n_slots, int min_rows,
-                           int max_rows, const F16Rows &x, float *out);
+                           int max_rows, const F16Rows &x, float *out, float *part = nullptr, int64_t part_floats = 0,
+                           const uint32_t *idx = nullptr);
 // The int8 path for experts with min_rows..max_rows rows, against int8 rows q
 // [n_rows, cols] (Q8_K for K-quants, Q8 for Q8_0; mode 0: the tokens' rows,
 // mode 1: the slots') with their block scales and 16-sums, as launch_moe_int.
@@ -303,7 +307,8 @@ hipError_t launch_f16_gemm_i8(hipStream_t st, int mode, int type, const ExpertTi
 // Plain GGUF rows: out [s_rows, rows]; with w_up (Q4_K) SwiGLU(w . x, w_up . x).
 // hipErrorNotSupported for other types, shapes or alignments.
 hipError_t launch_f16_gemm_plain(hipStream_t st, int type, const uint8_t *w, int64_t rows, int64_t cols,
-                                 const F16Rows &x, int64_t s_rows, float *out, const uint8_t *w_up = nullptr);
+                                 const F16Rows &x, int64_t s_rows, float *out, const uint8_t *w_up = nullptr,
+                                 float *part = nullptr, int64_t part_floats = 0);
 
 // ---- routing (kmoe_route.hip)
 // logits [S, E] = router [E, d] . x [S, d] in the reference's summation order

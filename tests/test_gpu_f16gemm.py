@@ -185,3 +185,36 @@ def test_int8_regime_expert_layers(ctx, E, k, d, F, S, gt, dt):
                 s, m = orc.q4k_block_acc(row, d, q.reshape(S, d)[tok], bs.reshape(S, -1)[tok])
                 assert np.array_equal(cap["up_sumi"].reshape(S * k, F, -1)[p, r], s)
                 assert np.array_equal(cap["up_mins"].reshape(S * k, F, -1)[p, r], m)
+
+
+# small grids: the columns split over work-groups (an even and an uneven last
+# part), one row tile per wave, plain and in the down product of few experts
+@pytest.mark.parametrize("t,rows,cols,S", [(Q4_K, 4100, 4096, 33), (Q6_K, 4096, 4352, 9), (Q8_0, 2052, 5056, 20),
+                                           (Q8_0, 2050, 4096, 17), (Q6_K, 8192, 1792, 64)])
+def test_column_split_plain(ctx, t, rows, cols, S):
+    from oracle import pyoracle as orc
+
+    w = random_blocks(t, rows, cols, seed=rows + cols)
+    x = np.random.default_rng(S).standard_normal((S, cols)).astype(np.float32)
+    w64 = orc.dequant(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    ref = x.astype(np.float64) @ w64.T
+    got = _matmul(ctx, t, w, rows, cols, x)
+    assert np.all(np.abs(got - ref) <= _bound(t, w64, x, cols))
+    assert rel_l2(got, ref) < 1e-6
+
+
+@pytest.mark.parametrize("dt,E,S", [(Q4_K, 3, 52), (Q6_K, 3, 52), (Q8_0, 4, 71)])
+def test_column_split_expert_down(ctx, dt, E, S):
+    import torch
+    from oracle import pyoracle as orc
+
+    d, F, k = 512, 2304, 2
+    spec = LayerSpec(E, k, d, F, Q4_K, seed=S + dt, down_type=dt, quantized=False)
+    x = orc.normal(S, S * d).reshape(S, d)
+    spec.upload(ctx, 2000 + dt)
+    n0 = ctx.profile_read("moe_down_f16")[1]
+    out = ctx.moe_ffn(2000 + dt, torch.from_numpy(x).cuda()).cpu().numpy()
+    assert ctx.profile_read("moe_down_f16")[1] == n0 + 1
+    layer = spec.oracle_layer()
+    assert np.bincount(layer.route(x)[0].ravel(), minlength=E).min() >= 4
+    assert rel_l2(out, layer.moe_ffn(x, 0)) < 3e-6
