@@ -165,7 +165,7 @@ struct F16Args {
   int n_expert;
   const uint8_t *pw, *pw2;  // plain: GGUF rows; with SwiGLU the gate and the up rows
   int64_t s_rows;           // plain: activation rows
-  int split_stages;         // columns split over blockIdx.y: stages per split (even; 0: no split), each split's
+  int split_stages;         // columns split over blockIdx.y: stages per split (even), each split's
   int64_t split_stride;     // sums at out + split * split_stride
   const float *ad;          // int8 rows: their block scales [.., cols / 256 or / 32]
   BlockDbg dbg;             // int8 rows with DBG: per-block integers (gate/down 0, up 1)
@@ -432,7 +432,8 @@ __device__ __forceinline__ bool find_block(const F16Args &a, int rblocks, int la
 // and Q8_0, so they are exact, and join y with the block scales as the int8
 // kernels do; Q6_K's sc * sum is rounded once per 16 columns. DBG adds the
 // exact integers to the capture (Q4_K, Q8_0).
-template <int T, int MODE, int RT, int NT, bool INT = false, bool DBG = false>
+// SPLIT: the columns over blockIdx.y (a form of its own: the bounds' registers).
+template <int T, int MODE, int RT, int NT, bool INT = false, bool DBG = false, bool SPLIT = false>
 __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   constexpr bool PLAIN = MODE >= 2, TILED = !PLAIN, SWIGLU = MODE == 0 || MODE == 3;
   static_assert(!SWIGLU || RT == 2, "gate and up tiles");
@@ -461,8 +462,8 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   const int64_t row_bytes = nb * (T == T_Q4_K ? 144 : T == T_Q6_K ? 210 : 34);
   const int64_t kp = (cols + 127) / 128 * 128;
   const int nst_all = (int)(kp / 128);
-  const int st_lo = a.split_stages ? (int)blockIdx.y * a.split_stages : 0;
-  const int nst = a.split_stages && st_lo + a.split_stages < nst_all ? st_lo + a.split_stages : nst_all;
+  const int st_lo = SPLIT ? (int)blockIdx.y * a.split_stages : 0;
+  const int nst = SPLIT && st_lo + a.split_stages < nst_all ? st_lo + a.split_stages : nst_all;
   const int64_t rbase = (int64_t)rb * RPB + wave * (SWIGLU ? 32 : 32 * RT);
   const uint8_t *wm[RT];  // matrix (uniform) and row offset of each tile (launch: a matrix is below 4 GiB)
   uint32_t wr[RT];
@@ -717,7 +718,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       const int tk = 32 * t + 8 * (v >> 2) + 4 * hh + (v & 3);
       if (tk >= nbt) continue;
       const int sh = INT ? 0 : -exs[tk];
-      float *o = a.out + (p0 + tok0 + tk) * rows + (SWIGLU ? 0 : (int64_t)blockIdx.y * a.split_stride);
+      float *o = a.out + (p0 + tok0 + tk) * rows + (SPLIT ? (int64_t)blockIdx.y * a.split_stride : 0);
       if constexpr (SWIGLU) {  // g / (1 + exp(-g)) * u
         const int64_t r = rbase + l32;
         const float gv = INT ? y[0][t][v] : ldexpf(y[0][t][v], sh), uv = INT ? y[1][t][v] : ldexpf(y[1][t][v], sh);
@@ -829,7 +830,7 @@ hipError_t launch_t(hipStream_t st, const F16Args &a, int64_t blocks, const Spli
       b.split_stride = stride;
       b.out = sp.part;
       ks = (nst + b.split_stages - 1) / b.split_stages;
-      KMOE_LAUNCH((k_f16_gemm<T, MODE, RT, NT, INT, DBG>), dim3(grid, (unsigned)ks), dim3(256), 0, st, b);
+      KMOE_LAUNCH((k_f16_gemm<T, MODE, RT, NT, false, false, true>), dim3(grid, (unsigned)ks), dim3(256), 0, st, b);
       hipLaunchKernelGGL(k_split_sum, dim3((unsigned)((stride / 4 + 255) / 256)), dim3(256), 0, st, sp.part, (int)ks,
                          stride, a.rows, stride / 4, a.out, MODE == 1 ? sp.idx : nullptr, a.rt.perm, a.rt.offsets,
                          a.min_rows);
