@@ -1033,8 +1033,9 @@ hipError_t launch_dispatch(hipStream_t st, const uint32_t *idx, int64_t n_slots,
                            uint32_t *offsets, uint32_t *inv, int32_t *n_active, int32_t *active, uint32_t *rank_tmp) {
   if (n_expert > kMaxExperts || n_expert <= 0) return hipErrorInvalidValue;
   // Many entries: a work-group per 1024, counts in rank_tmp (n_slots words;
-  // chunks x E of them, at most half as many for E <= 512). 4096 entries, 8
-  // experts: about 8 us either way.
+  // chunks x E of them). One work-group takes 6.6-6.9 us for 1024 entries of 8
+  // experts, 8.2 us for 1218 of 64 and 36-40 us for 14216 of 128; the two
+  // launches 16 us for those.
   const int64_t chunks = (n_slots + kDispChunk - 1) / kDispChunk;
   if (rank_tmp && n_slots >= 4096 && chunks * n_expert <= n_slots && chunks <= 65535) {
     KMOE_LAUNCH(k_dispatch_count, dim3((unsigned)chunks), dim3(256), 0, st, idx, n_slots, n_expert, rank_tmp);
