@@ -4,7 +4,7 @@ Transformer::forward (transformer.rs:278-302, 330-467, 591-631)."""
 import numpy as np
 import pytest
 
-from tests.helpers import (DSV2LITE, F32, Q4_K, Q6_K, Q8_0, LayerSpec, decoder_model, random_blocks, rel_l2,
+from tests.helpers import (DSV2LITE, F32, MOE6B, Q4_K, Q6_K, Q8_0, LayerSpec, decoder_model, random_blocks, rel_l2,
                            row_bytes, stack_model)
 
 pytestmark = pytest.mark.gpu
@@ -644,3 +644,39 @@ def test_norm_moe_ffn_rejects_null_rows(ctx, orc):
         assert not host(out).any()
     finally:
         ctx.layer_destroy(lid)
+
+
+@pytest.mark.parametrize("regime", [2, 0])
+def test_stack_with_a_long_prompt_matches_oracle(ctx, orc, regime):
+    """Two moe-6b-shaped layers, a 96-token prompt (the matrix-core prompt
+    attention and products) and single-token steps, each call's logits against
+    the oracle's Transformer. The bounds are those of
+    test_decoder_forward_matches_oracle: where activations are rounded to int8
+    on the way, an f32 difference of one ulp moves the logits by about 1.5%
+    (the oracle's own do, with 64 norm weights nudged by one ulp), so the exact
+    regime, where none are, carries the tight bound."""
+    from kestrel_amd.decoder import Decoder
+
+    rng = np.random.default_rng(31)
+    hp, T = stack_model(MOE6B, rng, n_ctx=104, n_layer=2, share=False)
+    ref = orc.Transformer(hp, T, regime=regime)
+    ctx.set_regime(regime)
+    ctx.profile_enable(True)
+    dec = Decoder(ctx, hp, T)
+    try:
+        n0 = [ctx.profile_read(n)[1] for n in ("f16_gemm", "moe_gate_up_f16")]
+        for i, toks in enumerate([rng.integers(0, MOE6B["vocab"], 96).tolist()] +
+                                 [[int(t)] for t in rng.integers(0, MOE6B["vocab"], 3)]):
+            a, b = host(dec.forward(toks)), ref.forward(toks)
+            scale = max(1.0, float(np.abs(b).max()))
+            md = float(np.abs(a - b).max())
+            if regime == 2:
+                assert rel_l2(a, b) < 1e-3 and md <= 2e-3 * scale, (i, rel_l2(a, b), md, scale)
+            else:
+                assert md <= 6e-2 * scale, (i, md, scale)
+            if i == 0:
+                assert all(ctx.profile_read(n)[1] > m for n, m in zip(("f16_gemm", "moe_gate_up_f16"), n0))
+    finally:
+        ctx.profile_enable(False)
+        ctx.set_regime(0)
+        dec.close()
