@@ -113,7 +113,9 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
   uint32_t vp[16][DL / 2];
   // key i of the lane's 16: the positions its score registers hold
   auto key = [&](int i) { return 8 * (i >> 2) + 4 * half + (i & 3); };
-  // Rows past n_max read as zeros: a block's buffer ends with its last row.
+  // Rows past n_max read as zeros: a block's buffer ends with its last row, and
+  // the row is in the lane's offset, which the bounds check covers (a scalar
+  // offset is not promised to be checked).
   const int ko = (int)((lane / CPR) * rowb) + 16 * (lane % CPR);
   const int vo = (int)(4 * half * rowb) + 2 * DL * l32;
   auto block = [&](const char *base, int b) {
@@ -123,21 +125,23 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
   };
   auto load_k = [&](int b) {
     const auto rs = block(kg, b);
+    int o = ko;
+    asm volatile("" : "+v"(o));  // formed here, not held in registers over the loop
 #pragma unroll
-    for (int i = 0; i < KPL; ++i)
-      kp[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, ko, (int)((64 / CPR) * i * rowb), 0);
+    for (int i = 0; i < KPL; ++i, o += (int)((64 / CPR) * rowb)) kp[i] = __builtin_amdgcn_raw_buffer_load_b128(rs, o, 0, 0);
   };
   auto load_v = [&](int b) {
     const auto rs = block(vg, b);
+    int o = vo;
+    asm volatile("" : "+v"(o));
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int so = (int)((8 * (i >> 2) + (i & 3)) * rowb);
+    for (int i = 0; i < 16; ++i, o += (int)((i & 3) ? rowb : 5 * rowb)) {  // row 8 * (i / 4) + i % 4
       if constexpr (DL == 4) {
-        const auto u = __builtin_amdgcn_raw_buffer_load_b64(rs, vo, so, 0);
+        const auto u = __builtin_amdgcn_raw_buffer_load_b64(rs, o, 0, 0);
         vp[i][0] = u[0];
         vp[i][1] = u[1];
       } else {
-        vp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, vo, so, 0);
+        vp[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, o, 0, 0);
       }
     }
   };

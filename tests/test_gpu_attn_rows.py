@@ -71,3 +71,20 @@ def test_values_that_are_not_finite_stay_in_the_rows_that_see_them(ctx):
     assert np.array_equal(np.isposinf(got), np.isposinf(ref)) and np.array_equal(np.isneginf(got), np.isneginf(ref))
     f = np.isfinite(ref)
     assert np.isinf(ref).any() and f.mean() > 0.9 and np.abs(got[f] - ref[f]).max() <= 1e-5 * max(1.0, np.abs(ref[f]).max())
+
+
+# the cache ends inside a key block (1, 5 and 31 rows of the last one), more
+# rows behind it in the same allocation: zeros there or NaN, the same bits
+@pytest.mark.parametrize("nh,nkv,hd,S,pos0", [(4, 2, 128, 33, 0), (4, 2, 64, 20, 17), (2, 2, 128, 70, 281)])
+def test_nothing_past_the_last_position_is_read(ctx, nh, nkv, hd, S, pos0):
+    from oracle import pyoracle as orc
+
+    rng = np.random.default_rng(S)
+    n = pos0 + S
+    kc, vc = (orc.f16_store(rng.standard_normal((n, nkv * hd))) for _ in range(2))
+    q = rng.standard_normal((S, nh * hd)).astype(np.float32)
+    got = [_run(ctx, q, np.concatenate([kc, t]), np.concatenate([vc, t]), nh, nkv, hd, pos0, n)
+           for t in (np.zeros((64, nkv * hd), np.uint16), np.full((64, nkv * hd), 0x7E00, np.uint16))]
+    assert np.array_equal(*(g.view(np.uint32) for g in got))
+    ref = orc.attention(q, kc, vc, nh, nkv, hd, pos0)
+    assert np.abs(got[1] - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
