@@ -1732,18 +1732,19 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
   const int f32_lo = regime == KMOE_REGIME_EXACT ? 1 : 4;
   const int f32_hi = (int)S;
   // The f16 matrix cores: x's pieces lie where y will (dead until the down
-  // product), their sums and exponents where h's int8 sums and scales will.
+  // product), their sums where h's int8 sums will, their exponents in the
+  // dispatch's scratch (a word per slot, dead after it).
   F16Rows xf;
   bool xf_done = false;
   if (any_f32) {
     const auto &SH = L->sh;
     const bool sh_q4 = SH.on && !int_path(regime, S) && SH.type[0] == KMOE_Q4_K && SH.type[1] == KMOE_Q4_K;
     int f32_done = 0;  // experts with f32_lo..f32_done rows are done
-    if (f16_experts(gt, d, F, slots) && f16_gemm_supported(gt, F, d, slots) && d % 128 == 0 && d <= 2 * k * F && k * F >= 32) {
+    if (f16_experts(gt, d, F, slots) && f16_gemm_supported(gt, F, d, slots) && d % 128 == 0 && d <= 2 * k * F) {
       xf.planes = (uint16_t *)w.y;
       xf.sums = gt == KMOE_Q4_K || sh_q4 ? (uint16_t *)w.hs : nullptr;
       xf.sums_stride = d / 8;
-      xf.ex = (int32_t *)w.hd;
+      xf.ex = (int32_t *)w.rank;
       const hipError_t e = timed(c, "split_f16", [&]() { return launch_split_f16(st, h, S, d, xf); });
       if (e == hipSuccess) xf_done = true;
       else if (e != hipErrorNotSupported) HIP_OK(c, e);
@@ -1817,15 +1818,16 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
   }
   if (any_f32) {
     int f32_done = 0;
-    // h's pieces in place; their sums and exponents in the slots' int8 sums and
-    // scales, which the f32 regime's slots do not use
+    // h's pieces in place; their sums in the slots' own int8 sums, which the f32
+    // regime's slots do not use, their exponents in the dispatch's scratch (not
+    // in the int8 scales: those of other slots lie there where blocks are wider
+    // than 32, and kmoe_moe_ffn_dbg hands them out)
     if (f16_down(dt, d, F, slots, max_active) && f16_gemm_supported(dt, d, F, slots) && F % 128 == 0) {
       F16Rows hf;
       hf.planes = (uint16_t *)w.h;
       hf.sums = dt == KMOE_Q4_K ? (uint16_t *)w.hs : nullptr;
       hf.sums_stride = F / 16 * 4;
-      hf.ex = (int32_t *)w.hd;
-      hf.ex_stride = F / 32;
+      hf.ex = (int32_t *)w.rank;
       hipError_t e = timed(c, "split_slots_f16", [&]() {
         return launch_split_f16(st, w.h, slots, F, hf, &rt, w.idx, f32_lo);
       });

@@ -218,3 +218,33 @@ def test_column_split_expert_down(ctx, dt, E, S):
     layer = spec.oracle_layer()
     assert np.bincount(layer.route(x)[0].ravel(), minlength=E).min() >= 4
     assert rel_l2(out, layer.moe_ffn(x, 0)) < 3e-6
+
+
+# AVX2 regime, experts of both kinds: the captured int8 rows of h are those of
+# the int path's slots, though the f32 regime's slots are split into pieces
+# before the capture is handed out
+@pytest.mark.parametrize("dt", [Q4_K, Q6_K, Q8_0])
+def test_capture_of_a_mixed_layer_keeps_the_int8_rows(ctx, dt):
+    import torch
+    from oracle import pyoracle as orc
+
+    E, k, d, F, S = 70, 3, 256, 512, 900  # 21 slots of experts with 1-3 rows, two of them 8 x another's number
+    spec = LayerSpec(E, k, d, F, Q4_K, seed=16, down_type=dt, zipf=0.5)
+    x = orc.normal(S, S * d).reshape(S, d) + np.float32(1.0)
+    spec.upload(ctx, 3000 + dt)
+    n0 = ctx.profile_read("moe_down_f16")[1]
+    _, cap = ctx.moe_ffn_dbg(3000 + dt, torch.from_numpy(x).cuda(), k, F, Q4_K, dt)
+    assert ctx.profile_read("moe_down_f16")[1] == n0 + 1
+    idx, _, perm, off = (t.cpu().numpy().astype(np.int64) for t in ctx.last_routing(S, k, E))
+    hq, hd, hs = (cap[n].cpu().numpy() for n in ("hq", "hd", "hs"))
+    seen = 0
+    for e in np.flatnonzero((np.diff(off) > 0) & (np.diff(off) < 4)):
+        p = np.arange(off[e], off[e + 1])
+        h = orc.swiglu(*(orc.matmul(Q4_K, w[e], F, d, x[perm[p] // k]) for w in (spec.gate, spec.up)))
+        q, sc = (orc.q8_quantize if dt == Q8_0 else orc.q8k_quantize)(h)[:2]
+        # (h in another float order: 1e-6 of it, which may move an int8 value across a rounding)
+        assert np.abs(hd[p] - np.asarray(sc).reshape(hd[p].shape)).max() <= 1e-5 * np.abs(sc).max()
+        assert np.abs(hq[p].astype(int) - np.asarray(q).reshape(hq[p].shape)).max() <= 1
+        assert np.array_equal(hs[p], hq[p].astype(np.int32).reshape(len(p), -1, 16).sum(2))
+        seen += len(p)
+    assert seen >= 8
