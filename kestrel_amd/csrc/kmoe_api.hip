@@ -121,17 +121,17 @@ bool f16_plain(int t, int64_t rows, int64_t cols, int64_t s_rows) {
   return t == KMOE_Q4_K ? s_rows >= 24 && (work >= 500e6 || outs >= 390000)
                         : s_rows >= 4 && (work >= 130e6 || outs >= 90000);
 }
-// The int8 regime's expert products. Q6_K and Q8_0 would otherwise run on dot4
+// The int8 regime's expert products: the fewest rows of an expert that takes the
+// f16 matrix cores (0: none do). Q6_K and Q8_0 would otherwise run on dot4
 // kernels; Q4_K has int8 matrix-core kernels, which pass over 128 rows of an
 // expert at a time and keep wide parts and few full experts. Layer, us, those
-// -> f16: Mixtral shape with Q6_K down 16 tokens 386 -> 776, 64 tokens 823 ->
-// 784, 512 tokens 5402 -> 1655, Q4_K down 512 tokens 965 -> 1049; DeepSeek-V2-
-// Lite shape (Q8_0 down) 64 tokens 341 -> 346, 128 tokens 413 -> 382; Qwen3
-// shape 128 tokens 186 -> 155, 1777 tokens 1389 -> 509; 32 experts of 1536 by
-// 2048, 400 tokens 169 -> 172, 1777 tokens 523 -> 402.
-bool f16_int(int t, int64_t E, int64_t d, int64_t F, int64_t slots, int64_t max_active) {
-  if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && slots >= (E >= 64 ? 1000 : 3000);
-  return slots >= (t == KMOE_Q6_K ? 16 : 8) * max_active;
+// -> f16, even routing: Mixtral shape with Q6_K down 48 tokens 678 -> 697, 64
+// tokens 809 -> 700, 512 tokens 5409 -> 1431; DeepSeek-V2-Lite shape (Q8_0 down)
+// 64 tokens 340 -> 350, 86 tokens 369 -> 369, 128 tokens 420 -> 385, 1777 tokens
+// 2696 -> 1961.
+int f16_int(int t, int64_t E, int64_t d, int64_t F, int64_t slots, int64_t max_active) {
+  if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && slots >= (E >= 64 ? 1000 : 3000) ? 1 : 0;
+  return slots >= (t == KMOE_Q6_K ? 16 : 8) * max_active ? 1 : 0;
 }
 // Expert layers, gate/up (whole layer, us): Mixtral shape 48 tokens 411 -> 488,
 // 64 tokens 656 -> 488 (both with the down product as below); Qwen3 shape 16
@@ -1679,6 +1679,32 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
       goto done;
     }
   }
+  // Experts of `lo` or more rows on the int path, gate/up (mode 0) or down: the
+  // f16 matrix cores (int8 regime; scratch for the pieces), the int8 ones, dot4.
+  auto int_many = [&](int mode, int t, int64_t rows, int64_t cols, int64_t n_rows, const int8_t *q, const float *qd,
+                      const int32_t *qs, uint8_t *scratch, float *o, int lo, const BlockDbg *g) -> int {
+    const bool mm = mfma && t == KMOE_Q4_K && moe_mfma_supported(rows, cols);
+    int hi = (int)S;
+    const int f16 = regime == KMOE_REGIME_INT8 && (mm || t != KMOE_Q4_K) ? f16_int(t, E, d, F, slots, max_active) : 0;
+    if (f16) {
+      const int from = f16 > lo ? f16 : lo;
+      const hipError_t e = timed(c, mode ? "moe_down_i8_f16" : "moe_gate_up_i8_f16", [&]() {
+        return launch_f16_gemm_i8(st, mode, t, tier, rows, cols, rt, (int)E, max_active, n_rows, slots, from, hi, q, qd,
+                                  qs, scratch, o, g);
+      });
+      if (e == hipSuccess) hi = from - 1;
+      else if (e != hipErrorNotSupported) HIP_OK(c, e);
+    }
+    if (lo > hi) return KMOE_OK;
+    if (mm) {
+      LAUNCH(c, mode ? "moe_down_mfma" : "moe_gate_up_mfma",
+             launch_moe_mfma(st, mode, tier, rows, cols, rt, regime, max_active, q, qd, qs, o, lo, hi, ring_rows, g));
+      return KMOE_OK;
+    }
+    LAUNCH(c, mode ? "moe_down_int" : "moe_gate_up_int",
+           launch_moe_int(st, mode, t, tier, rows, cols, rt, regime, max_active, S, q, qd, qs, o, lo, g));
+    return KMOE_OK;
+  };
   // Experts with a few rows on the int path (decode batches), tiled Q4_K:
   // the few-rows kernels; experts with more rows take the kernels after them.
   const bool small_ok = S >= 2;
@@ -1706,24 +1732,9 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
     }
     // AVX2 regime: experts of 4 or more rows are the f32 path's
     const bool more_int = regime == KMOE_REGIME_INT8 || small_rows < 3;
-    if (S > small_rows && more_int) {
-      hipError_t e = hipErrorNotSupported;
-      // the f16 matrix cores (x's piece and sums where y will be) ...
-      if (regime == KMOE_REGIME_INT8 && f16_int(gt, E, d, F, slots, max_active) && (!gd || f16_gemm_i8_captures(gt)))
-        e = timed(c, "moe_gate_up_i8_f16", [&]() {
-          return launch_f16_gemm_i8(st, 0, gt, tier, F, d, rt, (int)E, max_active, S, slots, small_rows + 1, (int)S, w.xq,
-                                    w.xd, w.xs, (uint8_t *)w.y, w.h, gd);
-        });
-      // ... or the int8 ones
-      if (e == hipErrorNotSupported && mfma && gt == KMOE_Q4_K)
-        e = timed(c, "moe_gate_up_mfma", [&]() {
-          return launch_moe_mfma(st, 0, tier, F, d, rt, regime, max_active, w.xq, w.xd, w.xs, w.h, small_rows + 1,
-                                 (int)S, ring_rows, gd);
-        });
-      if (e != hipErrorNotSupported) HIP_OK(c, e);
-      else
-        LAUNCH(c, "moe_gate_up_int", launch_moe_int(st, 0, gt, tier, F, d, rt, regime, max_active, S, w.xq, w.xd,
-                                                    w.xs, w.h, small_rows + 1, gd));
+    if (S > small_rows && more_int) {  // x's piece and sums lie where y will be
+      rc = int_many(0, gt, F, d, S, w.xq, w.xd, w.xs, (uint8_t *)w.y, w.h, small_rows + 1, gd);
+      if (rc) return rc;
     }
   }
   // The f32 regime's experts (quant.rs:242-260): tiled Q4_K rows stream
@@ -1797,23 +1808,9 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
       if (e == hipSuccess) small_rows = kFewRows;
       else if (e != hipErrorNotSupported) HIP_OK(c, e);
     }
-    if (S > small_rows && (regime == KMOE_REGIME_INT8 || small_rows < 3)) {
-      hipError_t e = hipErrorNotSupported;
-      // (h's piece and sums over its f32 rows, which this regime reads no more)
-      if (regime == KMOE_REGIME_INT8 && f16_int(dt, E, d, F, slots, max_active) && (!dd || f16_gemm_i8_captures(dt)))
-        e = timed(c, "moe_down_i8_f16", [&]() {
-          return launch_f16_gemm_i8(st, 1, dt, tier, d, F, rt, (int)E, max_active, slots, slots, small_rows + 1, (int)S,
-                                    w.hq, w.hd, w.hs, (uint8_t *)w.h, w.y, dd);
-        });
-      if (e == hipErrorNotSupported && mfma && dt == KMOE_Q4_K)
-        e = timed(c, "moe_down_mfma", [&]() {
-          return launch_moe_mfma(st, 1, tier, d, F, rt, regime, max_active, w.hq, w.hd, w.hs, w.y, small_rows + 1,
-                                 (int)S, ring_rows, dd);
-        });
-      if (e != hipErrorNotSupported) HIP_OK(c, e);
-      else
-        LAUNCH(c, "moe_down_int", launch_moe_int(st, 1, dt, tier, d, F, rt, regime, max_active, S, w.hq, w.hd,
-                                                 w.hs, w.y, small_rows + 1, dd));
+    if (S > small_rows && (regime == KMOE_REGIME_INT8 || small_rows < 3)) {  // h's, over its f32 rows, read no more
+      rc = int_many(1, dt, d, F, slots, w.hq, w.hd, w.hs, (uint8_t *)w.h, w.y, small_rows + 1, dd);
+      if (rc) return rc;
     }
   }
   if (any_f32) {

@@ -168,7 +168,8 @@ struct F16Args {
   int split_stages;         // columns split over blockIdx.y: stages per split (even), each split's
   int64_t split_stride;     // sums at out + split * split_stride
   const float *ad;          // int8 rows: their block scales [.., cols / 256 or / 32]
-  BlockDbg dbg;             // int8 rows with DBG: per-block integers (gate/down 0, up 1)
+  BlockDbg dbg;             // int8 rows with DBG: per-block integers (gate/down 0, up 1),
+  const int32_t *s16;       // the rows' 16-sums (Q6_K)
 };
 
 __device__ __forceinline__ void lds_dma16(const void *g, uint8_t *lds_wave_base) {
@@ -246,8 +247,8 @@ __device__ __forceinline__ uint32_t and_or(uint32_t a, uint32_t m, uint32_t o) {
 
 // Weights of the stage as MFMA operands (f16, exact): Q4_K sc*q (<= 945),
 // Q8_0 q, Q6_K q - 32; g: the f32 factor of each group (Q4_K d, Q8_0 d, Q6_K
-// d*sc as dequant_row forms it).
-template <int T, bool TILED>
+// d*sc as dequant_row forms it; INT: the bits of the integer sc).
+template <int T, bool TILED, bool INT>
 __device__ __forceinline__ void unpack(const Raw<T> &w, int64_t st, int64_t nb, h8 (&o)[8], float (&g)[kGroups<T>]) {
   uint32_t r[8][4];
   if constexpr (T == T_Q4_K) {
@@ -302,7 +303,8 @@ __device__ __forceinline__ void unpack(const Raw<T> &w, int64_t st, int64_t nb, 
     for (int s = 0; s < 8; ++s) {
       const int row = s >> 1, j = s & 1;
       const uint32_t sw = s < 4 ? w.sc.x : w.sc.y;
-      g[s] = d * (float)(int8_t)(sw >> (8 * (s & 3)));
+      const int sc = (int8_t)(sw >> (8 * (s & 3)));
+      g[s] = INT ? __builtin_bit_cast(float, sc) : d * (float)sc;
       // the nibbles of 32-row `row` and its 2 high bits
       const u32x2 nv = TILED ? w.n[row >> 1][j] : w.n[row & 1][j], qv = TILED ? w.q[row >> 1] : w.q[j];
       const int ns = TILED ? 4 * (row & 1) : 4 * (row >> 1), qs = TILED ? 4 * j + 2 * (row & 1) : 2 * row;
@@ -428,11 +430,25 @@ __device__ __forceinline__ bool find_block(const F16Args &a, int rblocks, int la
 // ends. Error against 64 bits: 3.1e-7 -> 1.8e-7 (Q4_K matrix).
 //
 // INT: int8 activation rows (the int8 path, quant.rs:262-281) as one exact f16
-// piece. A stage's sums are integers below 2^24 for Q4_K (128 * 15*63 * 127)
-// and Q8_0, so they are exact, and join y with the block scales as the int8
-// kernels do; Q6_K's sc * sum is rounded once per 16 columns. DBG adds the
-// exact integers to the capture (Q4_K, Q8_0).
+// piece. The MFMAs' sums are integers below 2^24 (Q4_K: 128 * 15*63 * 127 per
+// stage), so exact, and join y once per superblock with the block scales, as
+// the int8 kernels do: Q4_K d * (both stages) - dmin * mins; Q6_K the int32
+// sum of sc * sum (mad_i24); Q8_0 the stage's four blocks first, the weight's
+// f16 scale times the integer before the activation's. Long rows' sums move to
+// LDS every kIntChain stages, so that no chain of roundings is longer than the
+// int8 kernels' (which run parts of a row in parallel): error of the down
+// product against 64 bits 7.3e-8 (Q4_K, 768 columns), 8.8e-8 (Q6_K, 14336),
+// 8.9e-8 (Q8_0, 1408), there 7.3e-8, 8.9e-8 and 8.9e-8. A superblock's sums take
+// the registers of two tiles: gate and up by one token tile, or down by two
+// token tiles with one weight tile per wave, which unpacks a weight once per 64
+// tokens (Mixtral shape, Q6_K down, 512 tokens 1666 -> 1401 us per layer).
+// DBG adds the exact integers to the capture (its kernels spill; they are not
+// timed).
 // SPLIT: the columns over blockIdx.y (a form of its own: the bounds' registers).
+// Stages per chain of roundings: 8 superblocks, or 4 sums of 4 blocks.
+template <int T>
+constexpr int kIntChain = T == T_Q8_0 ? 4 : 16;
+
 template <int T, int MODE, int RT, int NT, bool INT = false, bool DBG = false, bool SPLIT = false>
 __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   constexpr bool PLAIN = MODE >= 2, TILED = !PLAIN, SWIGLU = MODE == 0 || MODE == 3;
@@ -445,6 +461,8 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   constexpr int ADW = T == T_Q8_0 ? 16 : 4, ADS = INT ? BN * ADW : 0;  // block scales of the stage's tokens
   __shared__ __attribute__((aligned(16))) uint8_t st0[NP * PLANE + ADS], st1[NP * PLANE + ADS + SUMS];
   __shared__ int exs[BN];
+  __shared__ float4 yl[INT ? 4 * RT * NT : 1][INT ? 256 : 1];  // each thread's own sums
+  static_assert(!INT || RT * NT == 2, "the registers of two tiles");
   const int tid = threadIdx.x, lane = tid & 63, hh = lane >> 5, l32 = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int e, rb, tb, n;
@@ -515,7 +533,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   // LDS offset of this lane's A piece of K step s: aoff ^ 32s
   const int aoff = 256 * l32 + 16 * (hh ^ (l32 & 15));
 
-  float y[RT][NT][16], z[RT][16];  // z: Q6_K with INT
+  float y[RT][NT][16];
 #pragma unroll
   for (int i = 0; i < RT; ++i)
 #pragma unroll
@@ -527,68 +545,106 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
 #pragma unroll
   for (int i = 0; i < RT; ++i) load_raw<T, TILED>(raw[i], wm[i], wr[i], nb, st_lo);
 
-  // INT: a group's sums P into y. Lane l's tokens of tile t are 8k + 4(l/32) + 0..3.
-  auto int_epilogue = [&](int t, int gi, f32x16 (&P)[RT], const uint8_t *cur, bool odd, int st,
-                          const float (&g)[RT][G], const h8 (&mo)[RT], const float (&dm)[RT]) {
+  // INT: sums on their way to y. Q4_K: the superblock's first half; Q8_0: the
+  // stage's blocks; Q6_K (as int): the superblock's sum of sc * (bits of P).
+  float z[INT ? RT : 1][NT][16];
+  int zi[INT && T == T_Q6_K ? RT : 1][NT][16];
+  // A group's sums P into y. Lane l's tokens of tile t are 8k + 4(l/32) + 0..3.
+  auto int_epilogue = [&](int t, int gi, f32x16 (&P)[RT], const uint8_t *cur, bool odd, int st, const float (&g)[RT][G],
+                          const h8 (&mo)[RT], const float (&dm)[RT]) {
     const uint8_t *ads = cur + NP * PLANE;
-    if constexpr (T == T_Q6_K) {  // z += sc * P over the stage, then y += ad * (d * z)
-#pragma unroll
-      for (int i = 0; i < RT; ++i)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          z[i][v] = gi == 0 ? g[i][gi] * P[i][v] : fmaf(g[i][gi], P[i][v], z[i][v]);
-          asm volatile("" : "+v"(z[i][v]));
-        }
-      if (gi < G - 1) return;
-    }
-    auto capture = [&](int i, int v, int32_t *const (&arr)[2], float val) {
+    auto capture = [&](int i, int v, int32_t *const (&arr)[2], int val) {
       const int tk = 32 * t + 8 * (v >> 2) + 4 * hh + (v & 3);
       const int64_t r = rbase + (SWIGLU ? 0 : 32 * i) + l32;
       if (tk < nbt && r < rows)
-        dbg_add(arr[SWIGLU ? i : 0], ((p0 + tok0 + tk) * rows + r) * nb + (T == T_Q8_0 ? 4 * st + gi : st >> 1), (int)val);
+        dbg_add(arr[SWIGLU ? i : 0], ((p0 + tok0 + tk) * rows + r) * nb + (T == T_Q8_0 ? 4 * st + gi : st >> 1), val);
     };
-    // (the minimum term in a pass of its own: its sums live beside P otherwise, and registers run out)
+    if constexpr (T == T_Q6_K) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      float sc[4];
-      if constexpr (T == T_Q8_0) {
+      for (int i = 0; i < RT; ++i) {
+        const int sc = __builtin_bit_cast(int, g[i][gi]);
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int p = sc * ((int)P[i][v] << 8 >> 8);
+          zi[i][t][v] = gi == 0 && !odd ? p : zi[i][t][v] + p;
+          asm volatile("" : "+v"(zi[i][t][v]));
+        }
+        if constexpr (DBG) {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int tk = 32 * t + 8 * (v >> 2) + 4 * hh + (v & 3);
+            const int o = sc * a.s16[src_row(tk) * (cols / 16) + 8 * st + gi];
+            capture(i, v, a.dbg.m, o);
+            capture(i, v, a.dbg.s, sc * (int)P[i][v] + 32 * o);
+          }
+        }
+      }
+      if (gi < G - 1 || !odd) return;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float sc[4];
+        *(float4 *)sc = *(const float4 *)(ads + 4 * (32 * t + 8 * k + 4 * hh));
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int v = 4 * k + c;
+            y[i][t][v] = fmaf(dm[i] * sc[c], (float)zi[i][t][v], y[i][t][v]);
+          }
+      }
+    } else if constexpr (T == T_Q8_0) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        float sc[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) sc[c] = *(const float *)(ads + 16 * (32 * t + 8 * k + 4 * hh + c) + 4 * gi);
-      } else {
-        *(float4 *)sc = *(const float4 *)(ads + 4 * (32 * t + 8 * k + 4 * hh));
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) {
+            const int v = 4 * k + c;
+            if constexpr (DBG) capture(i, v, a.dbg.s, (int)P[i][v]);
+            const float f = g[i][gi] * P[i][v];  // an f16 times a small integer: hardly rounded
+            z[i][t][v] = gi == 0 ? sc[c] * f : fmaf(sc[c], f, z[i][t][v]);
+            if (gi == G - 1) y[i][t][v] += z[i][t][v];
+            asm volatile("" : "+v"(z[i][t][v]));
+          }
+      }
+    } else {
+      if constexpr (DBG) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) capture(i, v, a.dbg.s, (int)P[i][v]);
+      }
+      if (!odd) {
+#pragma unroll
+        for (int i = 0; i < RT; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            z[i][t][v] = P[i][v];
+            asm volatile("" : "+v"(z[i][t][v]));
+          }
+        return;
       }
 #pragma unroll
-      for (int i = 0; i < RT; ++i)
+      for (int i = 0; i < RT; ++i) {
+        const h8 sm = *(const h8 *)(cur + NP * PLANE + ADS + 1024 * t + 32 * l32 + 16 * hh);
+        f32x16 M;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const int v = 4 * k + c;
-          if constexpr (DBG) capture(i, v, a.dbg.s, P[i][v]);
-          if constexpr (T == T_Q8_0) y[i][t][v] = fmaf(sc[c] * g[i][gi], P[i][v], y[i][t][v]);
-          else if constexpr (T == T_Q6_K) y[i][t][v] = fmaf(sc[c], z[i][v], y[i][t][v]);
-          else y[i][t][v] = fmaf(sc[c], g[i][gi] * P[i][v], y[i][t][v]);
-          asm volatile("" : "+v"(y[i][t][v]));
-        }
-    }
-    if constexpr (T == T_Q4_K) {
-      if (odd) {
+        for (int v = 0; v < 16; ++v) M[v] = 0.0f;
+        M = __builtin_amdgcn_mfma_f32_32x32x16_f16(sm, mo[i], M, 0, 0, 0);
 #pragma unroll
-        for (int i = 0; i < RT; ++i) {
-          const h8 sm = *(const h8 *)(cur + NP * PLANE + ADS + 1024 * t + 32 * l32 + 16 * hh);
-          f32x16 M;
+        for (int k = 0; k < 4; ++k) {
+          float sc[4];
+          *(float4 *)sc = *(const float4 *)(ads + 4 * (32 * t + 8 * k + 4 * hh));
 #pragma unroll
-          for (int v = 0; v < 16; ++v) M[v] = 0.0f;
-          M = __builtin_amdgcn_mfma_f32_32x32x16_f16(sm, mo[i], M, 0, 0, 0);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) {
-            float sc[4];
-            *(float4 *)sc = *(const float4 *)(ads + 4 * (32 * t + 8 * k + 4 * hh));
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-              const int v = 4 * k + c;
-              if constexpr (DBG) capture(i, v, a.dbg.m, M[v]);
-              y[i][t][v] = fmaf(-sc[c], dm[i] * M[v], y[i][t][v]);
-              asm volatile("" : "+v"(y[i][t][v]));
-            }
+          for (int c = 0; c < 4; ++c) {
+            const int v = 4 * k + c;
+            if constexpr (DBG) capture(i, v, a.dbg.m, (int)M[v]);
+            const float x = fmaf(g[i][gi], z[i][t][v] + P[i][v], -(dm[i] * M[v]));
+            y[i][t][v] = fmaf(sc[c], x, y[i][t][v]);
+            asm volatile("" : "+v"(y[i][t][v]));
           }
         }
       }
@@ -637,7 +693,8 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
           dm[i] = f16_bits_to_f32(raw[i].hd.x >> 16);
         }
       }
-      unpack<T, TILED>(raw[i], st, nb, w[i], g[i]);
+      if constexpr (T == T_Q6_K && INT) dm[i] = f16_bits_to_f32(raw[i].d);
+      unpack<T, TILED, INT>(raw[i], st, nb, w[i], g[i]);
 #pragma unroll
       for (int s = 0; s < 8; ++s) asm volatile("" : "+v"(w[i][s]));  // unpacked here, before raw is loaded again
     }
@@ -710,6 +767,31 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   for (int st = st_lo; st < nst; st += 2) {
     stage(st, st0, st1, false);
     if (st + 1 < nst) stage(st + 1, st1, st0, true);
+    if constexpr (INT) {  // (see kIntChain)
+      if ((st & (kIntChain<T> - 1)) == kIntChain<T> - 2 && st + 2 < nst) {
+#pragma unroll
+        for (int j = 0; j < 4 * RT * NT; ++j) {
+          float *yv = &y[j / (4 * NT)][j / 4 % NT][4 * (j % 4)];
+          float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+          if (st >= kIntChain<T>) v = yl[j][tid];
+          yl[j][tid] = make_float4(v.x + yv[0], v.y + yv[1], v.z + yv[2], v.w + yv[3]);
+          yv[0] = yv[1] = yv[2] = yv[3] = 0.0f;
+        }
+      }
+    }
+  }
+  if constexpr (INT) {
+    if (nst > kIntChain<T>) {
+#pragma unroll
+      for (int j = 0; j < 4 * RT * NT; ++j) {
+        float *yv = &y[j / (4 * NT)][j / 4 % NT][4 * (j % 4)];
+        const float4 v = yl[j][tid];
+        yv[0] += v.x;
+        yv[1] += v.y;
+        yv[2] += v.z;
+        yv[3] += v.w;
+      }
+    }
   }
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
@@ -852,12 +934,16 @@ hipError_t launch_grouped_t(hipStream_t st, int mode, const F16Args &a, int64_t 
   }
   const bool wide = n_slots > 32 * (int64_t)max_active;
   const int64_t blocks = n_slots / (wide ? 64 : 32) + ne;
-  if constexpr (T == T_Q6_K) {  // a scale per 16 columns: two token tiles need more registers than there are
+  if constexpr (INT) {  // (two tiles)
+    if (mode == 1 && wide) return launch_t<T, 1, 1, 2, INT, DBG>(st, a, blocks);
+  }
+  // one token tile: Q6_K's scale per 16 columns and the int8 rows' sums take the registers of two
+  if constexpr (T == T_Q6_K || INT) {
     return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne)
                      : launch_t<T, 1, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne, sp);
   } else {
-  if (wide) return mode == 0 ? launch_t<T, 0, 2, 2, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 2, INT, DBG>(st, a, blocks, sp);
-  return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, blocks) : launch_t<T, 1, 2, 1, INT, DBG>(st, a, blocks, sp);
+    if (wide) return mode == 0 ? launch_t<T, 0, 2, 2>(st, a, blocks) : launch_t<T, 1, 2, 2>(st, a, blocks, sp);
+    return mode == 0 ? launch_t<T, 0, 2, 1>(st, a, blocks) : launch_t<T, 1, 2, 1>(st, a, blocks, sp);
   }
 }
 
@@ -926,14 +1012,12 @@ hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier 
   }
 }
 
-bool f16_gemm_i8_captures(int type) { return type == T_Q4_K || type == T_Q8_0; }
-
 hipError_t launch_f16_gemm_i8(hipStream_t st, int mode, int type, const ExpertTier &tier, int64_t rows, int64_t cols,
                               const Routing &rt, int n_expert, int max_active, int64_t n_rows, int64_t n_slots,
                               int min_rows, int max_rows, const int8_t *q, const float *ad, const int32_t *s16,
                               uint8_t *scratch, float *out, const BlockDbg *dbg) {
   if (!f16_gemm_supported(type, rows, cols, n_slots) || cols % 128 || min_rows < 1 || ((uintptr_t)q & 15u) ||
-      ((uintptr_t)ad & 15u) || ((uintptr_t)scratch & 15u) || (dbg && !f16_gemm_i8_captures(type)))
+      ((uintptr_t)ad & 15u) || ((uintptr_t)scratch & 15u))
     return hipErrorNotSupported;
   if (max_active <= 0 || max_rows < min_rows) return hipSuccess;
   const int64_t n16 = n_rows * (cols / 16);
@@ -952,10 +1036,14 @@ hipError_t launch_f16_gemm_i8(hipStream_t st, int mode, int type, const ExpertTi
   a.max_rows = max_rows;
   a.n_expert = n_expert;
   a.ad = ad;
+  a.s16 = s16;
   if (dbg) {
     a.dbg = *dbg;
-    return type == T_Q4_K ? launch_grouped_t<T_Q4_K, true, true>(st, mode, a, n_slots, max_active)
-                          : launch_grouped_t<T_Q8_0, true, true>(st, mode, a, n_slots, max_active);
+    switch (type) {
+      case T_Q4_K: return launch_grouped_t<T_Q4_K, true, true>(st, mode, a, n_slots, max_active);
+      case T_Q6_K: return launch_grouped_t<T_Q6_K, true, true>(st, mode, a, n_slots, max_active);
+      default: return launch_grouped_t<T_Q8_0, true, true>(st, mode, a, n_slots, max_active);
+    }
   }
   switch (type) {
     case T_Q4_K: return launch_grouped_t<T_Q4_K, true>(st, mode, a, n_slots, max_active);

@@ -295,11 +295,10 @@ hipError_t launch_f16_gemm(hipStream_t st, int mode, int type, const ExpertTier 
 // The int8 path for experts with min_rows..max_rows rows, against int8 rows q
 // [n_rows, cols] (Q8_K for K-quants, Q8 for Q8_0; mode 0: the tokens' rows,
 // mode 1: the slots') with their block scales and 16-sums, as launch_moe_int.
-// scratch: i8_scratch_bytes(n_rows, cols), 16-byte aligned. dbg only where
-// f16_gemm_i8_captures. hipErrorNotSupported (nothing launched) otherwise and
+// scratch: i8_scratch_bytes(n_rows, cols), 16-byte aligned.
+// hipErrorNotSupported (nothing launched) for other types or alignments and
 // for cols % 128 != 0.
 constexpr int64_t i8_scratch_bytes(int64_t n_rows, int64_t cols) { return n_rows * cols * 2 + n_rows * (cols / 8); }
-bool f16_gemm_i8_captures(int type);
 hipError_t launch_f16_gemm_i8(hipStream_t st, int mode, int type, const ExpertTier &tier, int64_t rows, int64_t cols,
                               const Routing &rt, int n_expert, int max_active, int64_t n_rows, int64_t n_slots,
                               int min_rows, int max_rows, const int8_t *q, const float *ad, const int32_t *s16,

@@ -248,3 +248,59 @@ def test_capture_of_a_mixed_layer_keeps_the_int8_rows(ctx, dt):
         assert np.array_equal(hs[p], hq[p].astype(np.int32).reshape(len(p), -1, 16).sum(2))
         seen += len(p)
     assert seen >= 8
+
+
+# the int8 regime's products on int8 rows are exact integers joined once per
+# block: the captured call gives the layer's own bits, the integers are the
+# oracle's, and the down product is within the roundings of its join. Rows past
+# one chain of roundings (17 superblocks), one and two token tiles.
+@pytest.mark.parametrize("gt,dt,E,S,F", [(Q6_K, Q6_K, 3, 60, 4352), (Q8_0, Q6_K, 6, 130, 512), (Q4_K, Q8_0, 3, 60, 4352),
+                                         (Q4_K, Q4_K, 5, 1600, 512), (Q6_K, Q8_0, 5, 33, 384)])
+def test_int8_regime_down_is_the_exact_integers(ctx, gt, dt, E, S, F):
+    import torch
+    from oracle import pyoracle as orc
+
+    d, k, lid = 256, 2, 4000 + 100 * gt + dt
+    spec = LayerSpec(E, k, d, F, gt, seed=S + dt, down_type=dt, quantized=False)
+    x = orc.normal(S, S * d).reshape(S, d)
+    spec.upload(ctx, lid)
+    xd = torch.from_numpy(x).cuda()
+    ctx.set_regime(1)
+    try:
+        n0 = ctx.profile_read("moe_down_i8_f16")[1]
+        out = ctx.moe_ffn(lid, xd).cpu().numpy()
+        assert ctx.profile_read("moe_down_i8_f16")[1] == n0 + 1
+        cap_out, cap = ctx.moe_ffn_dbg(lid, xd, k, F, gt, dt)
+        idx, wsel, perm, off = (t.cpu().numpy() for t in ctx.last_routing(S, k, E))
+    finally:
+        ctx.set_regime(0)
+    assert np.array_equal(out.view(np.uint32), cap_out.cpu().numpy().view(np.uint32))
+    hq, hd, hs, si, mi = (cap[n].cpu().numpy() for n in ("hq", "hd", "hs", "down_sumi", "down_mins"))
+    y, mag = np.zeros((2, S * k, d))
+    size, at = {Q4_K: (144, 0), Q6_K: (210, 208), Q8_0: (34, 0)}[dt]
+    for e in range(E):
+        b = spec.down[e].reshape(d, -1, size)
+        half = lambda i: b[:, :, i:i + 2].copy().view(np.float16)[:, :, 0].astype(np.float64)
+        for p in range(int(off[e]), int(off[e + 1])):
+            for r in (0, 100, d - 1) if dt != Q8_0 else ():
+                acc = orc.q4k_block_acc if dt == Q4_K else orc.q6k_block_acc
+                s, m = acc(b[r].reshape(-1), F, hq[p], hs[p])
+                assert np.array_equal(si[p, r], s) and np.array_equal(mi[p, r], m)
+            if dt == Q8_0:
+                q = b[:, :, 2:].copy().view(np.int8).astype(np.int64)
+                assert np.array_equal(si[p], (q * hq[p].reshape(1, -1, 32)).sum(2))
+            t = si[p] * half(at) * hd[p]
+            if dt != Q8_0:
+                u = mi[p] * (half(2) if dt == Q4_K else 32 * half(at)) * hd[p]
+                if dt == Q4_K:  # the minimum term is rounded by itself
+                    mag[p] += np.abs(u).sum(1)
+                t = t - u
+            y[p], mag[p] = t.sum(1), mag[p] + np.abs(t).sum(1)
+    order = np.empty(S * k, np.int64)
+    order[perm.view(np.uint32).astype(np.int64)] = np.arange(S * k)
+    w = wsel.astype(np.float64).reshape(S, k, 1)
+    ref, bound = ((v[order].reshape(S, k, d) * w).sum(1) for v in (y, mag))
+    # roundings on one element's way: 3 in its term, chains of 8 (Q8_0: 4 and 4), of the parts and of the k slots
+    n = 3 + 8 + F // 2048 + 1 + k + (F // 512 if dt == Q8_0 else 0)
+    assert np.all(np.abs(out - ref) <= n * 2.0 ** -24 * bound)
+    assert rel_l2(out, ref) < 1.5e-7
