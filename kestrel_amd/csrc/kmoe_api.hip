@@ -122,15 +122,27 @@ bool f16_plain(int t, int64_t rows, int64_t cols, int64_t s_rows) {
                         : s_rows >= 4 && (work >= 130e6 || outs >= 90000);
 }
 // The int8 regime's expert products: the fewest rows of an expert that takes the
-// f16 matrix cores (0: none do). Q6_K and Q8_0 would otherwise run on dot4
-// kernels; Q4_K has int8 matrix-core kernels, which pass over 128 rows of an
-// expert at a time and keep wide parts and few full experts. Layer, us, those
-// -> f16, even routing: Mixtral shape with Q6_K down 48 tokens 678 -> 697, 64
-// tokens 809 -> 700, 512 tokens 5409 -> 1431; DeepSeek-V2-Lite shape (Q8_0 down)
-// 64 tokens 340 -> 350, 86 tokens 369 -> 369, 128 tokens 420 -> 385, 1777 tokens
-// 2696 -> 1961.
-int f16_int(int t, int64_t E, int64_t d, int64_t F, int64_t slots, int64_t max_active) {
-  if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && slots >= (E >= 64 ? 1000 : 3000) ? 1 : 0;
+// f16 matrix cores (0: none do). Layer, us.
+// Q6_K and Q8_0 would otherwise run on dot4 kernels (those -> f16, even
+// routing): Mixtral shape with Q6_K down 48 tokens 678 -> 697, 64 tokens 809 ->
+// 700, 512 tokens 5409 -> 1431; DeepSeek-V2-Lite shape (Q8_0 down) 64 tokens 340
+// -> 350, 86 tokens 369 -> 369, 128 tokens 420 -> 385, 1777 tokens 2696 -> 1961.
+// Q4_K has int8 matrix-core kernels with the same arithmetic and bits. They pass
+// over an expert's rows 128 at a time in one work-group per 128 weight rows, so
+// a ragged layer waits for its fullest expert; below one token tile they read
+// the weights once with less work. All experts there -> those of more than 32
+// rows here: Qwen3 shape (Zipf 1.1) 200 tokens 240 -> 186, 1777 tokens 1241 ->
+// 602, evenly routed 300 tokens 202 -> 207, 1024 tokens 390 -> 430, 2048 tokens
+// 645 -> 669; 32 experts of 1536 by 2048, even, 400 tokens 167 -> 171, 2048
+// tokens 542 -> 530, Zipf 1.1, 400 tokens 292 -> 216, 1200 tokens 744 -> 387.
+// Wider parts fill the chip with one expert's work-groups: 32 of 1536 by 4096,
+// 512 tokens even 349 -> 379, Zipf 1 411 -> 419; 16 of 4096 by 2048, 512 tokens
+// even 332 -> 419, Zipf 1 404 -> 442; Mixtral shape 512 tokens 984 -> 1172.
+// In calls of few tokens the launches decide: Qwen3 shape 48 tokens 139 -> 148,
+// 64 tokens 144 -> 150, 96 tokens 168 -> 160.
+constexpr int kF16IntRows = 33, kF16IntTokens = 96;
+int f16_int(int t, int64_t d, int64_t F, int64_t S, int64_t slots, int64_t max_active) {
+  if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && S >= kF16IntTokens ? kF16IntRows : 0;
   return slots >= (t == KMOE_Q6_K ? 16 : 8) * max_active ? 1 : 0;
 }
 // Expert layers, gate/up (whole layer, us): Mixtral shape 48 tokens 411 -> 488,
@@ -1685,7 +1697,7 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
                       const int32_t *qs, uint8_t *scratch, float *o, int lo, const BlockDbg *g) -> int {
     const bool mm = mfma && t == KMOE_Q4_K && moe_mfma_supported(rows, cols);
     int hi = (int)S;
-    const int f16 = regime == KMOE_REGIME_INT8 && (mm || t != KMOE_Q4_K) ? f16_int(t, E, d, F, slots, max_active) : 0;
+    const int f16 = regime == KMOE_REGIME_INT8 && (mm || t != KMOE_Q4_K) ? f16_int(t, d, F, S, slots, max_active) : 0;
     if (f16) {
       const int from = f16 > lo ? f16 : lo;
       const hipError_t e = timed(c, mode ? "moe_down_i8_f16" : "moe_gate_up_i8_f16", [&]() {

@@ -255,7 +255,7 @@ def test_capture_of_a_mixed_layer_keeps_the_int8_rows(ctx, dt):
 # oracle's, and the down product is within the roundings of its join. Rows past
 # one chain of roundings (17 superblocks), one and two token tiles.
 @pytest.mark.parametrize("gt,dt,E,S,F", [(Q6_K, Q6_K, 3, 60, 4352), (Q8_0, Q6_K, 6, 130, 512), (Q4_K, Q8_0, 3, 60, 4352),
-                                         (Q4_K, Q4_K, 5, 1600, 512), (Q6_K, Q8_0, 5, 33, 384)])
+                                         (Q4_K, Q4_K, 4, 150, 4352), (Q6_K, Q8_0, 5, 33, 384)])
 def test_int8_regime_down_is_the_exact_integers(ctx, gt, dt, E, S, F):
     import torch
     from oracle import pyoracle as orc
@@ -278,6 +278,7 @@ def test_int8_regime_down_is_the_exact_integers(ctx, gt, dt, E, S, F):
     hq, hd, hs, si, mi = (cap[n].cpu().numpy() for n in ("hq", "hd", "hs", "down_sumi", "down_mins"))
     y, mag = np.zeros((2, S * k, d))
     size, at = {Q4_K: (144, 0), Q6_K: (210, 208), Q8_0: (34, 0)}[dt]
+    assert dt != Q4_K or np.diff(off.astype(np.int64)).max() > 32  # (fewer rows: the int8 kernels)
     for e in range(E):
         b = spec.down[e].reshape(d, -1, size)
         half = lambda i: b[:, :, i:i + 2].copy().view(np.float16)[:, :, 0].astype(np.float64)
