@@ -29,15 +29,17 @@ __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t 
   lo = __builtin_bit_cast(uint32_t, l);
 }
 
-// exp(x) * 2^14 for x <= 0 (or NaN): 2^n * 2^f with n the nearest integer of
-// x * log2(e) and f the rest, the product carried to twice the precision.
+// exp(x) * 2^14 for x <= 0 (or NaN). x = n ln 2 + r with n the nearest integer,
+// ln 2 taken off in two parts (the argument reduction of Cody and Waite,
+// Software Manual for the Elementary Functions, 1980; the first part leaves no
+// rounding), so r is good to 2^-26 and exp(x) = 2^n * 2^(r / ln 2).
 __device__ __forceinline__ float exp14(float x) {
+  constexpr double ln2 = 0.69314718055994530942;
+  constexpr float ln2hi = (float)ln2, ln2lo = (float)(ln2 - (double)ln2hi), inv = (float)(1.0 / ln2);
   x = x < -150.0f ? -150.0f : x;
-  const float c = 0x1.715476p+0f, cc = 0x1.4ae0bep-26f;  // log2(e) = c + cc
-  const float ph = x * c;
-  const float pl = fmaf(x, cc, fmaf(x, c, -ph));
-  const float n = rintf(ph);
-  return ldexpf(__builtin_amdgcn_exp2f((ph - n) + pl), (int)n + 14);
+  const float n = rintf(x * inv);
+  const float r = fmaf(n, -ln2lo, fmaf(n, -ln2hi, x));
+  return ldexpf(__builtin_amdgcn_exp2f(r * inv), (int)n + 14);
 }
 
 __device__ __forceinline__ void wave_lds_order() {
