@@ -17,14 +17,16 @@ typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int kQT = 32;  // query rows per work-group
 constexpr int kKB = 32;  // key positions per block
 
-// A pair of f32 as two dwords of f16 pairs: hi (toward zero) and lo, the
-// nearest f16 of what hi leaves. x = hi + lo to 2^-23 of x for |x| in
-// 2^-2..2^15 and to 2^-25 below that.
+// A pair of f32 as two dwords of f16 pairs: hi, the nearest f16, and lo, the
+// nearest f16 of 2^12 times what hi leaves. x = hi + lo * 2^-12 to 2^-23 of x
+// for |x| in 2^-14..2^15 and to 2^-37 below that. (Without the 2^12, lo's
+// exponent ends at 2^-25: elements some 2^20 below their row's largest, or
+// softmax weights so far below a first position's, would lose their bits.)
+constexpr float kLo = 0x1p-12f;
 __device__ __forceinline__ void split2(float a, float b, uint32_t &hi, uint32_t &lo) {
-  const auto h = __builtin_amdgcn_cvt_pkrtz(a, b);
-  h2 l;
-  l.x = (_Float16)(a - (float)h[0]);
-  l.y = (_Float16)(b - (float)h[1]);
+  const h2 h = {(_Float16)a, (_Float16)b};
+  const h2 l = {(_Float16)fmaf((float)h.x, -1.0f / kLo, a * (1.0f / kLo)),
+                (_Float16)fmaf((float)h.y, -1.0f / kLo, b * (1.0f / kLo))};
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, l);
 }
@@ -73,9 +75,11 @@ __device__ __forceinline__ void wave_lds_order() {
 // the small pieces, and to rows before its position), so a result that is not
 // finite is formed again from its row's own positions, in plain f32.
 // Measured on MI355X (16 heads of 128 over 4, 777 rows after 611 positions):
-// the work-group per (row, 64 positions) of attn_batch takes 2450 us, bound by
-// its per-row loads, hand-offs and VALU products; this kernel 33 us
-// (errors against 64 bits 2.1e-7 and 2.1e-7).
+// the work-group per (row, 64 positions) of attn_batch takes 2400 us, bound by
+// its per-row loads, hand-offs and VALU products; this kernel 31.6 us, bound by
+// the softmax's VALU work between the two products. Error against 64 bits 2.2e-7
+// there, 1.9e-7 here; where all but e^-20 of the weight lies on a position with a
+// zero value, 6.1e-7 in both.
 template <int HD, int NW>
 __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const float *__restrict__ q, const uint16_t *__restrict__ kc,
                                                       const uint16_t *__restrict__ vc, int64_t s_rows, int nh,
@@ -182,7 +186,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
     if (c == 0) ml[0][r] = ldexpf(1.0f / sqrtf((float)HD), -sh);
   }
   lds_barrier();
-  const float fs = ml[0][l32];
+  const float fs = ml[0][l32], fsl = fs * kLo;
   lds_barrier();
   f32x16 O[DL];
 #pragma unroll
@@ -207,7 +211,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
     float mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      float t = fmaf(Sh[0][i] + Sh[1][i], fs, S[i] * fs);
+      float t = fmaf(Sh[0][i] + Sh[1][i], fs, S[i] * fsl);
       if (edge) t = b * kKB + key(i) < n_me ? t : -INFINITY;
       S[i] = t;
       mx = fmaxf(mx, t);
@@ -244,9 +248,13 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
     for (int t = 0; t < DL; ++t) {
       f32x16 T = f32x16{0};
 #pragma unroll
-      for (int st = 0; st < 4; ++st)
-        T = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[st & 1][t]),
-                                                   __builtin_bit_cast(h8, st < 2 ? pl[st & 1] : ph[st & 1]), T, 0, 0, 0);
+      for (int st = 0; st < 2; ++st)
+        T = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[st][t]), __builtin_bit_cast(h8, pl[st]), T, 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) T[i] *= kLo;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+        T = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, a[st][t]), __builtin_bit_cast(h8, ph[st]), T, 0, 0, 0);
 #pragma unroll
       for (int i = 0; i < 16; ++i) O[t][i] = fmaf(O[t][i], f, T[i]);
     }

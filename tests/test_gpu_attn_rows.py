@@ -88,3 +88,33 @@ def test_nothing_past_the_last_position_is_read(ctx, nh, nkv, hd, S, pos0):
     assert np.array_equal(*(g.view(np.uint32) for g in got))
     ref = orc.attention(q, kc, vc, nh, nkv, hd, pos0)
     assert np.abs(got[1] - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
+
+
+# bits far below a row's largest: a first position that takes all but e^-20 of
+# the weight and has a zero value, and a q element 2^24 above the others whose
+# K is zero; what is left keeps f32's bits
+@pytest.mark.parametrize("kind,hd", [("sink", 128), ("sink", 64), ("outlier", 128), ("outlier", 64)])
+def test_small_weights_and_elements_keep_their_bits(ctx, kind, hd):
+    rng = np.random.default_rng(hd)
+    nh, nkv, S, pos0 = 4, 2, 70, 90
+    n = pos0 + S
+    q = rng.standard_normal((S, nh, hd)).astype(np.float32)
+    k, v = (rng.standard_normal((n, nkv, hd)).astype(np.float16) for _ in range(2))
+    if kind == "sink":
+        q[:, :, 0] = 8.0
+        k[:, :, 0] = 0.0
+        k[0] = 0.0
+        k[0, :, 0] = 20 * np.sqrt(hd) / 8.0
+        v[0] = 0.0
+    else:
+        q[:, :, 3] = 2.0 ** 24
+        k[:, :, 3] = 0.0
+    got = _run(ctx, q.reshape(S, -1), k.view(np.uint16).reshape(n, -1), v.view(np.uint16).reshape(n, -1), nh, nkv, hd,
+               pos0, n).reshape(S, nh, hd)
+    for s in range(S):
+        for h in range(nh):
+            sc = k[:pos0 + s + 1, h // 2].astype(np.float64) @ q[s, h].astype(np.float64) / np.sqrt(hd)
+            e = np.exp(sc - sc.max())
+            ref = e @ v[:pos0 + s + 1, h // 2].astype(np.float64) / e.sum()
+            # an f32 score is off by up to |score| 2^-23, and as much of its weight (20 at the sink)
+            assert np.linalg.norm(got[s, h] - ref) <= (3e-6 if kind == "sink" else 1.5e-6) * np.linalg.norm(ref)
