@@ -400,9 +400,14 @@ int kmoe_kv_store(kmoe_ctx *ctx, const float *k_dev, const float *v_dev, int64_t
  * queries q [s_rows, n_head, head_dim] (after RoPE) over the f16 caches
  * [n_ctx, n_kv * head_dim]; query s attends positions 0 ..= position(s),
  * head h reads kv head h / (n_head / n_kv). out [s_rows, n_head * head_dim].
- * Scores use quant::dot's summation order (bit-identical); the softmax is
- * taken over chunks of 64 positions and merged, within 1e-6 relative of the
- * reference's single pass. head_dim 64 or 128, at most 16 query heads per
+ * Calls of fewer than 16 rows, and caches that are not 16-byte aligned: scores
+ * use quant::dot's summation order (bit-identical), the softmax is taken over
+ * chunks of 64 positions and merged. From 16 rows (prompt chunks) scores and
+ * weighted values are formed on the matrix cores, q and the softmax weights as
+ * two f16 pieces of 23 bits together, with f32 sums in another order: a row's
+ * last bits then depend on the number of rows in its call (how a prompt is cut),
+ * not on n_ctx or on where the position is kept. Either way within 1e-6 relative
+ * of the reference's single pass. head_dim 64 or 128, at most 16 query heads per
  * kv head. */
 int kmoe_attention(kmoe_ctx *ctx, const float *q_dev, const uint16_t *k_cache_dev, const uint16_t *v_cache_dev,
                    int64_t s_rows, int32_t n_head, int32_t n_kv, int32_t head_dim, int64_t pos0,

@@ -16,6 +16,10 @@ typedef float f32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 constexpr int kQT = 32;  // query rows per work-group
 constexpr int kKB = 32;  // key positions per block
+// Calls that end at most here run four waves per work-group, whichever form was
+// launched: a row's bits do not depend on the cache's capacity or on where its
+// position is kept.
+constexpr int kNarrow = 8 * kKB;
 
 // A pair of f32 as two dwords of f16 pairs: hi, the nearest f16, and lo, the
 // nearest f16 of 2^12 times what hi leaves. x = hi + lo * 2^-12 to 2^-23 of x
@@ -51,7 +55,7 @@ __device__ __forceinline__ void wave_lds_order() {
 }
 
 // Work-group: NW waves, one query head, 32 query rows; wave w takes the key
-// blocks w, w + NW, ... (32 positions each) with its own running softmax, and
+// blocks w, w + nw, ... (32 positions each) with its own running softmax, and
 // the waves are merged through LDS in wave order. NW = 4, two work-groups per
 // CU, or 8 (see launch_attn_rows).
 //
@@ -112,6 +116,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
   };
   const int n_me = visible(s0 + l32), n_first = visible(s0), n_max = visible(s0 + kQT - 1);
   const int nblk = (n_max + kKB - 1) / kKB;
+  const int nw = NW == 4 || pos + s_rows > kNarrow ? NW : 4;
   const int64_t rowb = (int64_t)nkv * HD * 2;  // bytes per position
   const char *kg = (const char *)(kc + (int64_t)g * HD), *vg = (const char *)(vc + (int64_t)g * HD);
 
@@ -151,7 +156,8 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
       }
     }
   };
-  if (wave < nblk) {
+  const int b0 = wave < nw ? wave : nblk;
+  if (b0 < nblk) {
     load_k(wave);
     load_v(wave);
   }
@@ -192,11 +198,11 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
 #pragma unroll
   for (int t = 0; t < DL; ++t) O[t] = f32x16{0};
   float m = -INFINITY, l = 0.0f;  // l and O times 2^14
-  for (int b = wave; b < nblk; b += NW) {
+  for (int b = b0; b < nblk; b += nw) {
 #pragma unroll
     for (int i = 0; i < KPL; ++i) L.a.k[wave][(64 / CPR) * i + lane / CPR][lane % CPR] = kp[i];
-    const bool more = b + NW < nblk;
-    if (more) load_k(b + NW);
+    const bool more = b + nw < nblk;
+    if (more) load_k(b + nw);
     wave_lds_order();
     f32x16 S = f32x16{0}, Sh[2] = {f32x16{0}, f32x16{0}};
 #pragma unroll
@@ -258,7 +264,7 @@ __global__ void __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) k_attn_rows(const fl
 #pragma unroll
       for (int i = 0; i < 16; ++i) O[t][i] = fmaf(O[t][i], f, T[i]);
     }
-    if (more) load_v(b + NW);
+    if (more) load_v(b + nw);
   }
   // merge the waves: element i of tile t is dim DL * key(i) + t of query l32
   lds_barrier();  // every wave is done with its K tile and q
@@ -342,8 +348,9 @@ hipError_t launch_attn_rows(hipStream_t st, const float *q, const uint16_t *kc, 
   // 8 waves per work-group where the grid has at most one per CU and the rows
   // see more than 8 blocks: 64 rows after 1000 positions, 32 heads 22.0 -> 17.7
   // us, 24 after 900, 16 heads 19.6 -> 16.4; but 16 rows after none 8.5 -> 10.2,
-  // where the larger merge is all that is added.
-  const bool wide = nh * tiles <= cus && (pos_dev ? n_ctx : pos0 + s_rows) > 8 * kKB;
+  // where the larger merge is all that is added. (With a position on the device
+  // the kernel finds out itself.)
+  const bool wide = nh * tiles <= cus && (pos_dev ? n_ctx : pos0 + s_rows) > kNarrow;
   if (hd == 64) {
     if (wide) KMOE_ATTN(64, 8);
     else KMOE_ATTN(64, 4);

@@ -118,3 +118,21 @@ def test_small_weights_and_elements_keep_their_bits(ctx, kind, hd):
             ref = e @ v[:pos0 + s + 1, h // 2].astype(np.float64) / e.sum()
             # an f32 score is off by up to |score| 2^-23, and as much of its weight (20 at the sink)
             assert np.linalg.norm(got[s, h] - ref) <= (3e-6 if kind == "sink" else 1.5e-6) * np.linalg.norm(ref)
+
+
+# a row's bits are the same for a position on the host or on the device, however
+# much longer than the call's positions the cache is (either side of 256)
+@pytest.mark.parametrize("nh,nkv,hd,S,pos0", [(4, 2, 128, 40, 100), (2, 2, 64, 33, 223), (4, 2, 128, 20, 400)])
+def test_bits_do_not_depend_on_the_cache_length(ctx, nh, nkv, hd, S, pos0):
+    import torch
+    from oracle import pyoracle as orc
+
+    rng = np.random.default_rng(S)
+    kc, vc = (orc.f16_store(rng.standard_normal((2000, nkv * hd))) for _ in range(2))
+    q = rng.standard_normal((S, nh * hd)).astype(np.float32)
+    pos = torch.tensor([pos0], dtype=torch.int32).cuda()
+    got = [_run(ctx, q, kc, vc, nh, nkv, hd, p, n, pos_dev=pd) for p, pd in ((pos0, None), (0, pos))
+           for n in (pos0 + S, 2000)]
+    assert all(np.array_equal(g.view(np.uint32), got[0].view(np.uint32)) for g in got)
+    ref = orc.attention(q, kc, vc, nh, nkv, hd, pos0)
+    assert np.abs(got[0] - ref).max() <= 1e-5 * max(1.0, np.abs(ref).max())
