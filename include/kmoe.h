@@ -352,7 +352,15 @@ int kmoe_moe_last_routing(kmoe_ctx *ctx, uint32_t *idx_dev, float *w_dev, uint32
  * full", EngineError::ContextFull, transformer.rs:278-282); with a device
  * position, rows past n_ctx are skipped by the kernels. A call that grows the
  * context's decoder workspace (kmoe_get_rows, and kmoe_attention at a larger
- * size) allocates: run one call of each size before capturing a graph. */
+ * size) allocates: run one call of each size before capturing a graph.
+ *
+ * kmoe_matmul, kmoe_norm_matmul and kmoe_attention_matmul of a few rows and more
+ * in the f32 regime keep scratch of their own for the matrix-core kernels (at
+ * most 4.2 bytes per activation and the partial sums of a small product). It
+ * counts against the VRAM budget, is given back when another allocation or a
+ * lower limit needs its bytes, and may grow inside a capture; the graph then
+ * holds it until the context ends. Only where the budget has no room for it do
+ * other kernels compute the product, slower and with other last bits. */
 
 /* quant::get_row (quant.rs:342-345) for the token embedding lookup
  * (transformer.rs:381-389): out[s] = row ids[s] of the GGUF table

@@ -192,6 +192,13 @@ struct kmoe_ctx {
   size_t dws_size = 0;
   uint8_t *aws = nullptr;
   size_t aws_size = 0, aws_counters = 0;
+  // scratch of the f16 products of quant::matmul (see pieces()), and outgrown
+  // ones that a captured graph holds
+  uint8_t *pws = nullptr;
+  size_t pws_size = 0;
+  bool pws_captured = false, pws_used = false, pws_wait = false;
+  hipEvent_t pws_event = nullptr;
+  std::vector<void *> pws_retired;
   // last moe_ffn routing (pointers into ws) and its sizes
   uint32_t *last_idx = nullptr, *last_perm = nullptr, *last_off = nullptr;
   float *last_w = nullptr;
@@ -233,8 +240,28 @@ struct DeviceGuard {
   }
 };
 
+bool capturing(hipStream_t s) {
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &cap) != hipSuccess) (void)hipGetLastError();
+  return cap != hipStreamCaptureStatusNone;
+}
+
+void release(kmoe_ctx *c, uint64_t bytes) { c->vram_reserved -= bytes < c->vram_reserved ? bytes : c->vram_reserved; }
+
+// Gives back the f16 products' scratch, unless a graph holds it.
+bool drop_pieces(kmoe_ctx *c) {
+  if (!c->pws || c->pws_captured || capturing(c->stream)) return false;
+  (void)hipStreamSynchronize(c->stream);
+  (void)hipFree(c->pws);  // (waits for the device: any stream it was used on)
+  release(c, c->pws_size);
+  c->pws = nullptr;
+  c->pws_size = 0;
+  return true;
+}
+
 // Ledger::reserve (ledger.rs:75-102): an error value, never an OOM.
 int reserve(kmoe_ctx *c, uint64_t bytes, const char *purpose) {
+  if (c->vram_reserved + bytes > c->vram_limit) drop_pieces(c);
   if (c->vram_reserved + bytes > c->vram_limit)
     return fail(c, KMOE_E_BUDGET,
                 "VRAM budget exhausted: requested %llu bytes for %s, %llu/%llu reserved",
@@ -243,12 +270,15 @@ int reserve(kmoe_ctx *c, uint64_t bytes, const char *purpose) {
   c->vram_reserved += bytes;
   return KMOE_OK;
 }
-void release(kmoe_ctx *c, uint64_t bytes) { c->vram_reserved -= bytes < c->vram_reserved ? bytes : c->vram_reserved; }
 
 int dev_alloc(kmoe_ctx *c, size_t bytes, void **p, const char *purpose) {
   int rc = reserve(c, bytes, purpose);
   if (rc) return rc;
   hipError_t e = hipMalloc(p, bytes ? bytes : 1);
+  if (e == hipErrorOutOfMemory && drop_pieces(c)) {
+    (void)hipGetLastError();
+    e = hipMalloc(p, bytes ? bytes : 1);
+  }
   if (e != hipSuccess) {
     release(c, bytes);
     return fail(c, KMOE_E_HIP, "hipMalloc(%zu) for %s: %s", bytes, purpose, hipGetErrorString(e));
@@ -551,14 +581,11 @@ struct QRows {
   int32_t *s;
   float *part;
   int64_t part_floats;
-  F16Rows xf;  // the f32 regime's activation pieces, over the same bytes (planes null: no room for them)
-  float *xf_part = nullptr;  // and the partial sums of their products
-  int64_t xf_part_floats = 0;
 };
 QRows carve_qrows(uint8_t *base, int64_t s_rows, int64_t cols, size_t *total, int64_t part_floats = 0) {
   Carver cv{base};
   QRows r{cv.take<int8_t>(s_rows * cols), cv.take<float>(s_rows * (cols / 32)), cv.take<int32_t>(s_rows * (cols / 16)),
-          nullptr, part_floats, F16Rows{}};
+          nullptr, part_floats};
   r.part = part_floats > 0 ? cv.take<float>(part_floats) : nullptr;
   *total = cv.off;
   return r;
@@ -578,39 +605,58 @@ F16Rows carve_f16(uint8_t *base, int64_t s_rows, int64_t cols, size_t *total) {
   return r;
 }
 
-// The scratch of one quant::matmul in the workspace: `need` bytes that it must
-// have (int8 rows, partial sums, more behind them) and, where the f16 matrix
-// cores can take the f32 regime, the activation pieces over the same bytes.
-// Those are left out (and the other f32 kernels run) where only they would
-// push the workspace past the VRAM budget, or grow it inside a graph capture.
-int matmul_ws(kmoe_ctx *c, int t, int64_t rows, int64_t s_rows, int64_t cols, int64_t part_floats, size_t need, QRows *qr) {
-  size_t f16 = 0;
-  int64_t pf = 0;
-  size_t pieces = 0;
-  if (f16_plain(t, rows, cols, s_rows) && f16_gemm_supported(t, rows, cols, s_rows)) {
-    pf = f16_gemm_part_floats(t, rows, cols, s_rows);
-    carve_f16(nullptr, s_rows, cols, &pieces);
-    f16 = pieces + align_up((size_t)pf * 4);
+// Scratch of one f16 product outside the expert layers: `need` bytes, or null
+// where the VRAM budget has no room for them (the other f32 kernels run then).
+// It is a buffer of its own: the workspace keeps what lies in it (the last
+// routing) and grows no further, and the buffer is given back when the budget
+// is short (drop_pieces). It grows inside a graph capture too, so that a call's
+// kernels depend on its sizes and not on the calls before it; a buffer that a
+// graph holds is kept until the context ends. A call on another stream than the
+// last one waits for that one's use (kmoe_set_stream).
+uint8_t *pieces(kmoe_ctx *c, size_t need) {
+  const bool cap = capturing(c->stream);
+  if (need > c->pws_size) {
+    const size_t sz = align_up(need + need / 4);
+    const bool keep = cap || c->pws_captured;
+    if (c->vram_reserved - (keep ? 0 : c->pws_size) + sz > c->vram_limit) return nullptr;
+    if (c->pws && keep) {
+      c->pws_retired.push_back(c->pws);
+      c->pws = nullptr;
+      c->pws_size = 0;
+    }
+    drop_pieces(c);
+    c->pws_captured = false;
+    void *p = nullptr;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (cap) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    const hipError_t e = hipMalloc(&p, sz);
+    if (cap) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    c->vram_reserved += sz;
+    c->pws = (uint8_t *)p;
+    c->pws_size = sz;
   }
-  size_t want = f16 > need ? f16 : need;
-  if (want > need && want > c->ws_size) {
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(c->stream, &cap) != hipSuccess) (void)hipGetLastError();
-    if (cap != hipStreamCaptureStatusNone ||
-        c->vram_reserved - c->ws_size + align_up(want + want / 4) > c->vram_limit)
-      want = need;
+  if (cap) c->pws_captured = true;
+  else if (c->pws_wait && hipStreamWaitEvent(c->stream, c->pws_event, 0) != hipSuccess) return nullptr;
+  else c->pws_wait = false;
+  c->pws_used = true;
+  return c->pws;
+}
+
+// The stream is about to change: what uses the pieces on the old one is marked.
+void leave_stream(kmoe_ctx *c, hipStream_t next) {
+  if (next == c->stream || !c->pws_used || capturing(c->stream) || capturing(next)) return;
+  DeviceGuard g(c->device);
+  if ((!c->pws_event && hipEventCreateWithFlags(&c->pws_event, hipEventDisableTiming) != hipSuccess) ||
+      hipEventRecord(c->pws_event, c->stream) != hipSuccess) {
+    (void)hipGetLastError();  // no such stream any more
+    return;
   }
-  int rc = ensure_ws(c, want);
-  if (rc && want > need) rc = ensure_ws(c, need);
-  if (rc) return rc;
-  size_t n = 0;
-  *qr = carve_qrows(c->ws, s_rows, cols, &n, part_floats);
-  if (f16 && f16 <= c->ws_size) {
-    qr->xf = carve_f16(c->ws, s_rows, cols, &n);
-    qr->xf_part = (float *)(c->ws + pieces);
-    qr->xf_part_floats = pf;
-  }
-  return KMOE_OK;
+  c->pws_wait = true;
+  c->pws_used = false;
 }
 
 // The f32 path's partial sums for the shared expert's three products.
@@ -622,8 +668,9 @@ int64_t sh_part_floats(int64_t Fs, int64_t d, int64_t S) {
 // quant::matmul (quant.rs:229-328) on validated arguments: F32 weights in the
 // reference's summation order; otherwise the context's regime picks the f32
 // GEMM or int8 activations (quantized into qr) and the int8 matvec.
+// own_scratch: the product may allocate (pieces()).
 int matmul_core(kmoe_ctx *c, int t, const uint8_t *w, int64_t rows, int64_t cols, const float *x, int64_t s_rows,
-                float *out, const QRows &qr, float *wf = nullptr) {
+                float *out, const QRows &qr, float *wf = nullptr, bool own_scratch = false) {
   if (xtype(t)) {  // F16, BF16, Q4_0, Q4_1, Q5_0, Q5_1, Q5_K
     const int64_t rb = bytes_for(t, cols);
     if (t == KMOE_F16 || t == KMOE_BF16 || !int_path(c->regime, s_rows)) {
@@ -646,17 +693,20 @@ int matmul_core(kmoe_ctx *c, int t, const uint8_t *w, int64_t rows, int64_t cols
   }
   if (!int_path(c->regime, s_rows)) {
     // the f16 matrix cores, where the activations' pieces have room
-    if (qr.xf.planes) {
-      F16Rows xf = qr.xf;
-      if (t != KMOE_Q4_K) xf.sums = nullptr;
-      hipError_t e = timed(c, "split_f16", [&]() { return launch_split_f16(c->stream, x, s_rows, cols, xf); });
-      if (e == hipSuccess)
-        e = timed(c, "f16_gemm", [&]() {
-          return launch_f16_gemm_plain(c->stream, t, w, rows, cols, xf, s_rows, out, nullptr, qr.xf_part,
-                                       qr.xf_part_floats);
-        });
-      if (e == hipSuccess) return KMOE_OK;
-      if (e != hipErrorNotSupported) HIP_OK(c, e);
+    if (own_scratch && f16_plain(t, rows, cols, s_rows) && f16_gemm_supported(t, rows, cols, s_rows) &&
+        ((uintptr_t)x & 15u) == 0 && ((uintptr_t)w & (t == KMOE_Q4_K ? 15u : 1u)) == 0) {
+      const int64_t pf = f16_gemm_part_floats(t, rows, cols, s_rows);
+      size_t n = 0;
+      carve_f16(nullptr, s_rows, cols, &n);
+      if (uint8_t *p = pieces(c, n + align_up((size_t)pf * 4))) {
+        size_t m = 0;
+        F16Rows xf = carve_f16(p, s_rows, cols, &m);
+        if (t != KMOE_Q4_K) xf.sums = nullptr;
+        LAUNCH(c, "split_f16", launch_split_f16(c->stream, x, s_rows, cols, xf));
+        LAUNCH(c, "f16_gemm", launch_f16_gemm_plain(c->stream, t, w, rows, cols, xf, s_rows, out, nullptr,
+                                                    (float *)(p + n), pf));
+        return KMOE_OK;
+      }
     }
     // Q4_K rows: the bf16-split kernel (exact products on the bf16 matrix
     // cores); other types, or unaligned buffers, the fp32 GEMM
@@ -759,6 +809,9 @@ int kmoe_destroy(kmoe_ctx *c) {
   if (c->hio) (void)hipFree(c->hio);
   if (c->dws) (void)hipFree(c->dws);
   if (c->aws) (void)hipFree(c->aws);
+  if (c->pws) (void)hipFree(c->pws);
+  for (void *p : c->pws_retired) (void)hipFree(p);
+  if (c->pws_event) (void)hipEventDestroy(c->pws_event);
   if (c->counters) (void)hipFree(c->counters);
   if (c->own) (void)hipStreamDestroy(c->own);
   delete c;
@@ -769,11 +822,13 @@ const char *kmoe_last_error(const kmoe_ctx *c) { return c ? c->err.c_str() : "nu
 
 int kmoe_set_stream(kmoe_ctx *c, void *s) {
   if (!c) return KMOE_E_INVALID;
+  leave_stream(c, (hipStream_t)s);
   c->stream = (hipStream_t)s;  // NULL is the null stream, not "our own"
   return KMOE_OK;
 }
 int kmoe_use_own_stream(kmoe_ctx *c) {
   if (!c) return KMOE_E_INVALID;
+  leave_stream(c, c->own);
   c->stream = c->own;
   return KMOE_OK;
 }
@@ -807,6 +862,10 @@ int kmoe_vram_set_limit(kmoe_ctx *c, uint64_t limit) {
     size_t fr = 0, tot = 0;
     HIP_OK(c, hipMemGetInfo(&fr, &tot));
     limit = tot;
+  }
+  if (limit < c->vram_reserved) {
+    DeviceGuard g(c->device);
+    drop_pieces(c);
   }
   if (limit < c->vram_reserved)
     return fail(c, KMOE_E_BUDGET, "limit %llu below the %llu bytes already reserved", (unsigned long long)limit,
@@ -973,11 +1032,12 @@ int kmoe_matmul(kmoe_ctx *c, int t, const void *w, size_t w_len, int64_t rows, i
   carve_qrows(nullptr, s_rows, cols, &need, pf);
   const size_t wf_off = need;
   if (staged) need = wf_off + align_up((size_t)rows * (size_t)cols * 4);
-  QRows qr{};
-  int rc = matmul_ws(c, t, rows, s_rows, cols, pf, need, &qr);
+  int rc = ensure_ws(c, need);
   if (rc) return rc;
+  size_t qn = 0;
+  QRows qr = carve_qrows(c->ws, s_rows, cols, &qn, pf);
   return matmul_core(c, t, (const uint8_t *)w, rows, cols, x, s_rows, out, qr,
-                     staged ? (float *)(c->ws + wf_off) : nullptr);
+                     staged ? (float *)(c->ws + wf_off) : nullptr, true);
 }
 
 int kmoe_matmul_host(kmoe_ctx *c, int t, const void *w, size_t w_len, int64_t rows, int64_t cols, const float *x,
@@ -2107,9 +2167,9 @@ int kmoe_norm_matmul(kmoe_ctx *c, float *x, const float *y, const float *norm_w,
   const int64_t pf = gemm_f32_part_floats(rows, cols, 1, s_rows, s_rows);
   size_t need = 0;
   carve_qrows(nullptr, s_rows, cols, &need, pf);
-  QRows qr{};
-  int rc = matmul_ws(c, t, rows, s_rows, cols, pf, need, &qr);
+  int rc = ensure_ws(c, need);
   if (rc) return rc;
+  QRows qr = carve_qrows(c->ws, s_rows, cols, &need, pf);
   if (t != KMOE_F32 && int_path(c->regime, s_rows) && rows > 0) {
     hipError_t e = timed(c, "rmsnorm_quant", [&]() {
       return launch_rmsnorm_quant(c->stream, x, y, norm_w, s_rows, cols, eps, h, is_kq(t), qr.q, qr.d, qr.s);
@@ -2119,7 +2179,7 @@ int kmoe_norm_matmul(kmoe_ctx *c, float *x, const float *y, const float *norm_w,
   }
   LAUNCH(c, "rmsnorm", launch_add_rmsnorm(c->stream, x, y, norm_w, s_rows, cols, eps, h));
   if (rows == 0) return KMOE_OK;
-  return matmul_core(c, t, (const uint8_t *)w, rows, cols, h, s_rows, out, qr);
+  return matmul_core(c, t, (const uint8_t *)w, rows, cols, h, s_rows, out, qr, nullptr, true);
 }
 
 // Position checks shared by rope, kv_store and attention: with a host
@@ -2228,15 +2288,15 @@ int kmoe_attention_matmul(kmoe_ctx *c, const float *q, const uint16_t *k_cache, 
   const int64_t pf = gemm_f32_part_floats(rows, cols, 1, s_rows, s_rows);
   size_t need = 0;
   carve_qrows(nullptr, s_rows, cols, &need, pf);
-  QRows qr{};
-  rc = matmul_ws(c, t, rows, s_rows, cols, pf, need, &qr);
+  rc = ensure_ws(c, need);
   if (rc) return rc;
+  QRows qr = carve_qrows(c->ws, s_rows, cols, &need, pf);
   bool done = false;
   rc = attention_rows(c, q, k_cache, v_cache, s_rows, n_head, n_kv, head_dim, pos0, pos_dev, n_ctx, attn, &done);
   if (rc) return rc;
   if (done) {
     if (rows == 0) return KMOE_OK;
-    return matmul_core(c, t, (const uint8_t *)w, rows, cols, attn, s_rows, out, qr);
+    return matmul_core(c, t, (const uint8_t *)w, rows, cols, attn, s_rows, out, qr, nullptr, true);
   }
   const int supers = attn_supers(pos_dev ? n_ctx : std::min(n_ctx, pos0 + s_rows));
   rc = ensure_aws(c, (size_t)s_rows * n_head, (size_t)attn_part_floats(s_rows, n_head, head_dim, supers) * 4);
@@ -2257,7 +2317,7 @@ int kmoe_attention_matmul(kmoe_ctx *c, const float *q, const uint16_t *k_cache, 
   LAUNCH(c, "attention", launch_attention(c->stream, q, k_cache, v_cache, s_rows, n_head, n_kv, head_dim, pos0,
                                           pos_dev, n_ctx, supers, part, counters, attn));
   if (rows == 0) return KMOE_OK;
-  return matmul_core(c, t, (const uint8_t *)w, rows, cols, attn, s_rows, out, qr);
+  return matmul_core(c, t, (const uint8_t *)w, rows, cols, attn, s_rows, out, qr, nullptr, true);
 }
 
 int kmoe_rope_kv_store(kmoe_ctx *c, const float *q, const float *k, const float *v, int64_t s_rows, int32_t n_head,

@@ -305,3 +305,124 @@ def test_int8_regime_down_is_the_exact_integers(ctx, gt, dt, E, S, F):
     n = 3 + 8 + F // 2048 + 1 + k + (F // 512 if dt == Q8_0 else 0)
     assert np.all(np.abs(out - ref) <= n * 2.0 ** -24 * bound)
     assert rel_l2(out, ref) < 1.5e-7
+
+
+def _product(S, rows=8192, cols=512, seed=5):
+    """A Q4_K product whose pieces are far larger than the int8 rows' workspace."""
+    import torch
+    from oracle import pyoracle as orc
+
+    w = torch.from_numpy(random_blocks(Q4_K, rows, cols, seed=seed)).cuda()
+    return w, rows, cols, torch.from_numpy(orc.normal(seed, S * cols).reshape(S, cols)).cuda()
+
+
+def test_products_leave_the_workspace_and_the_last_routing_alone(ctx):
+    import torch
+
+    S, d = 300, 512
+    spec = LayerSpec(6, 2, d, 256, Q4_K, seed=3, quantized=False)
+    spec.upload(ctx, 5000)
+    w, rows, cols, x = _product(S)
+    gen = []
+    for _ in range(2):  # (the second time nothing grows)
+        ctx.moe_ffn(5000, x)
+        before = [t.cpu().numpy().copy() for t in ctx.last_routing(S, 2, 6)]
+        ctx.matmul(Q4_K, w, rows, cols, x)
+        gen.append(ctx.workspace_generation())
+    assert gen[0] == gen[1]
+    assert all(np.array_equal(a, b.cpu().numpy()) for a, b in zip(before, ctx.last_routing(S, 2, 6)))
+
+
+def test_scratch_of_products_gives_way_to_other_allocations():
+    from kestrel_amd.kmoe import REGIME_INT8, Context
+
+    w, rows, cols, x = _product(600)
+    c = Context(0)
+    c.profile_enable(True)
+    try:
+        c.set_regime(REGIME_INT8)  # int8 rows: no pieces
+        c.matmul(Q4_K, w, rows, cols, x)
+        base = c.vram_usage()[0]
+        c.set_regime(0)
+        full = c.matmul(Q4_K, w, rows, cols, x).cpu().numpy()
+        assert c.vram_usage()[0] > base and c.profile_read("f16_gemm")[1] == 1
+        E, d, F = 12, 256, 256
+        room = c.vram_usage()[0] - base
+        c.vram_set_limit(c.vram_usage()[0] + room // 4)
+        assert room // 4 < 3 * E * F * 144 < room  # more than is free, less than with the pieces' bytes
+        c.layer_create(0, E, 1, d, F, Q4_K, Q4_K, Q4_K)
+        again = c.matmul(Q4_K, w, rows, cols, x).cpu().numpy()  # no room for the pieces now
+        assert c.profile_read("f16_gemm")[1] == 1 and rel_l2(again, full) < 2e-6
+        c.layer_destroy(0)
+        assert np.array_equal(c.matmul(Q4_K, w, rows, cols, x).cpu().numpy(), full)
+        c.vram_set_limit(base)  # a lower limit takes them too
+        assert c.vram_usage()[0] == base
+    finally:
+        c.close()
+
+
+def test_a_product_first_called_in_a_capture_runs_the_same_kernels():
+    """Nothing before the capture but the int8 workspace: the graph holds the
+    matrix-core product, its replays give the eager bits, and a larger eager
+    product between replays leaves the graph's scratch alone."""
+    import torch
+    from kestrel_amd.kmoe import REGIME_INT8, Context
+
+    w, rows, cols, x = _product(200)
+    wl, _, _, xl = _product(900, seed=6)
+    c = Context(0)
+    c.profile_enable(True)
+    want = c.matmul(Q4_K, w, rows, cols, x).cpu().numpy()
+    want_l = c.matmul(Q4_K, wl, rows, cols, xl).cpu().numpy()
+    c.close()
+    c = Context(0)
+    try:
+        c.set_regime(REGIME_INT8)
+        c.matmul(Q4_K, w, rows, cols, x)
+        c.matmul(Q4_K, wl, rows, cols, xl)
+        c.set_regime(0)
+        out = torch.empty((200, rows), device="cuda")
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        try:
+            with torch.cuda.graph(g):
+                c.set_stream(torch.cuda.current_stream())
+                out.copy_(c.matmul(Q4_K, w, rows, cols, x))
+        finally:
+            c.set_stream(torch.cuda.current_stream())
+        for i in range(4):
+            out.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(out.cpu().numpy().view(np.uint32), want.view(np.uint32)), i
+            t = (wl, xl, want_l) if i % 2 == 0 else (w, x, want)
+            assert np.array_equal(c.matmul(Q4_K, t[0], rows, cols, t[1]).cpu().numpy(), t[2])
+        torch.cuda.synchronize()
+        del g
+    finally:
+        c.close()
+
+
+def test_products_on_two_streams_do_not_share_pieces_at_once():
+    import torch
+    from kestrel_amd.kmoe import Context
+
+    rows, cols, S = 4096, 4096, 512
+    w, _, _, _ = _product(1, rows, cols)
+    xs = [torch.randn(S, cols, device="cuda", generator=torch.Generator("cuda").manual_seed(i)) for i in range(2)]
+    c = Context(0)
+    try:
+        want = [c.matmul(Q4_K, w, rows, cols, x).clone() for x in xs]
+        st = [torch.cuda.Stream(), torch.cuda.Stream()]
+        outs = [torch.empty((8, S, rows), device="cuda") for _ in range(2)]
+        torch.cuda.synchronize()
+        for i in range(8):
+            for j in range(2):
+                c.set_stream(st[j])
+                c.check(c.lib.kmoe_matmul(c.h, Q4_K, w.data_ptr(), w.numel(), rows, cols, xs[j].data_ptr(), S,
+                                          outs[j][i].data_ptr()))
+        torch.cuda.synchronize()
+        assert all(torch.equal(outs[j][i], want[j]) for j in range(2) for i in range(8))
+    finally:
+        torch.cuda.synchronize()
+        c.close()
