@@ -20,14 +20,16 @@ typedef uint32_t u32x2a2 __attribute__((ext_vector_type(2), aligned(2)));
 //
 // A row is scaled by a power of two so that its largest finite magnitude lies
 // in [2^14, 2^15), and each element becomes two f16 pieces: hi, the nearest
-// f16, and lo, the nearest f16 of what hi leaves. x = hi + lo to 2^-23 of x,
-// and to 2^-40 of the row's largest element for elements too small for that.
+// f16, and lo, the nearest f16 of 2^12 times what hi leaves (a factor of its
+// own: lo's exponent would end 2^-39 below the row's largest otherwise, and
+// elements some 2^20 below it lose their bits). x = hi + lo * 2^-12 to 2^-23 of
+// x, and to 2^-51 of the row's largest element for elements too small for that.
 // (An infinity keeps hi = inf, lo = 0.) Row r of the result is cols hi pieces,
 // then cols lo pieces (cols rounded up to 128, the rest zeros): the row's own
 // size in f32, so rows whose length is a multiple of 128 convert in place.
 // Inside every 8 elements the order is 0,2,1,3,4,6,5,7, the order in which
 // the weights' 4-bit pairs come out of a dword. For Q4_K's minimum term the
-// sums of 32 scaled elements, times 2^-5, go to `sums` as two f16 pieces: per
+// sums of 32 scaled elements, times 2^-5, go to `sums` as two such pieces: per
 // 256 elements 8 hi pieces, then 8 lo.
 struct SplitArgs {
   const float *x;
@@ -38,6 +40,8 @@ struct SplitArgs {
   const uint32_t *idx, *perm, *offsets;
   int min_rows;
 };
+
+constexpr float kLo = 0x1p-12f;  // the lo pieces' unit
 
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
   h2 v;
@@ -100,7 +104,7 @@ __global__ void __launch_bounds__(64 * WV) k_split_f16(SplitArgs a) {
     for (int k = 0; k < 8; ++k) {
       const float y = ldexpf(t[k], sh);
       hf[k] = (float)(_Float16)y;
-      lf[k] = fabsf(y) < __builtin_inff() ? y - hf[k] : 0.0f;
+      lf[k] = fabsf(y) < __builtin_inff() ? (y - hf[k]) * (1.0f / kLo) : 0.0f;
       s += y;
     }
     *(u32x4 *)(hi + c) = u32x4{pack_h2(hf[0], hf[2]), pack_h2(hf[1], hf[3]), pack_h2(hf[4], hf[6]), pack_h2(hf[5], hf[7])};
@@ -109,7 +113,7 @@ __global__ void __launch_bounds__(64 * WV) k_split_f16(SplitArgs a) {
       s = ldexpf(group_sum<4>(s), -5);
       if ((tid & 3) == 0) {
         const _Float16 sh16 = (_Float16)s;
-        const _Float16 sl16 = (_Float16)(fabsf(s) < __builtin_inff() ? s - (float)sh16 : 0.0f);
+        const _Float16 sl16 = (_Float16)(fabsf(s) < __builtin_inff() ? (s - (float)sh16) * (1.0f / kLo) : 0.0f);
         _Float16 *p = (_Float16 *)(sums + c / 256 * 32) + (c / 32 % 8);
         p[0] = sh16;
         p[8] = sl16;
@@ -149,7 +153,7 @@ __global__ void __launch_bounds__(256) k_i8_f16(const int8_t *__restrict__ q, co
     _Float16 *p = (_Float16 *)((uint8_t *)sums + r * sums_stride + c / 256 * 32) + (c / 32 % 8);
     const _Float16 hi = (_Float16)s;
     p[0] = hi;
-    p[8] = (_Float16)(s - (float)hi);
+    p[8] = (_Float16)((s - (float)hi) * (1.0f / kLo));
   }
 }
 
@@ -325,16 +329,17 @@ __device__ __forceinline__ void unpack(const Raw<T> &w, int64_t st, int64_t nb, 
   for (int s = 0; s < 8; ++s) o[s] = __builtin_bit_cast(h8, u32x4{r[s][0], r[s][1], r[s][2], r[s][3]});
 }
 
-// The 8 minimums of a Q4_K superblock, times 32, as the MFMA's B operand (both
-// K halves: against the sums' hi and lo pieces).
+// The 8 minimums of a Q4_K superblock, times 32, as the MFMA's B operand (the K
+// halves: against the sums' hi and lo pieces).
 __device__ __forceinline__ h8 mins_operand(const u32x4 &hd) {
   h8 o;
+  const float f = (threadIdx.x & 32) ? 32.0f * kLo : 32.0f;
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     int sA, mA, sB, mB;
     q4k_scale_min_pair(hd.y, hd.z, hd.w, k, sA, mA, sB, mB);
-    o[2 * k] = (_Float16)((float)mA * 32.0f);
-    o[2 * k + 1] = (_Float16)((float)mB * 32.0f);
+    o[2 * k] = (_Float16)((float)mA * f);
+    o[2 * k + 1] = (_Float16)((float)mB * f);
   }
   return o;
 }
@@ -732,6 +737,8 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       if (T != T_Q4_K && t == 1) next_weights();  // two tiles and these types' larger stage: registers
       if (t >= ntt) break;
       f32x16 P[RT];
+      uint32_t lo2 = 0x0c000c00u;  // two f16 kLo, opaque per tile (products of both tiles' would be kept in registers)
+      asm volatile("" : "+s"(lo2));
 #pragma unroll
       for (int j = 0; j < NR; ++j) {
         if (j < NR - 1) read(t, j + 1);
@@ -747,7 +754,19 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
               for (int v = 0; v < 16; ++v) P[i][v] = 0.0f;
           }
 #pragma unroll
-          for (int i = 0; i < RT; ++i) P[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[j & 1][u], w[i][s], P[i], 0, 0, 0);
+          for (int i = 0; i < RT; ++i) {
+            h8 wv = w[i][s];
+            // the lo pieces' unit: in the weights (still exact in f16), or Q4_K, whose
+            // small products are all summed first, in their sum
+            if constexpr (T != T_Q4_K) {
+              if (!INT && pl_of(j, u) == 1) wv *= __builtin_bit_cast(h8, u32x4{lo2, lo2, lo2, lo2});
+            }
+            P[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[j & 1][u], wv, P[i], 0, 0, 0);
+            if (!INT && T == T_Q4_K && j == 1 && u == 3) {
+#pragma unroll
+              for (int v = 0; v < 16; ++v) P[i][v] *= kLo;
+            }
+          }
           if (INT && last_of(j, u)) {
             int_epilogue(t, gi, P, cur, odd, st, g, mo, dm);
           } else if (last_of(j, u)) {  // its last
@@ -942,7 +961,10 @@ hipError_t launch_grouped_t(hipStream_t st, int mode, const F16Args &a, int64_t 
     return mode == 0 ? launch_t<T, 0, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne)
                      : launch_t<T, 1, 2, 1, INT, DBG>(st, a, n_slots / 32 + ne, sp);
   } else {
-    if (wide) return mode == 0 ? launch_t<T, 0, 2, 2>(st, a, blocks) : launch_t<T, 1, 2, 2>(st, a, blocks, sp);
+    // (Q8_0: two by two tiles spill 31 registers; DeepSeek-V2-Lite shape, 1777
+    // tokens 1077 us per layer so, 1001 with one weight tile per wave)
+    constexpr int RT = T == T_Q8_0 ? 1 : 2;
+    if (wide) return mode == 0 ? launch_t<T, 0, 2, 2>(st, a, blocks) : launch_t<T, 1, RT, 2>(st, a, blocks, sp);
     return mode == 0 ? launch_t<T, 0, 2, 1>(st, a, blocks) : launch_t<T, 1, 2, 1>(st, a, blocks, sp);
   }
 }
@@ -955,7 +977,7 @@ struct PlainShape {
 };
 PlainShape plain_shape(int type, int64_t rows, int64_t s_rows) {
   const int64_t cus = num_cus(), r2 = (rows + 255) / 256, n64 = (s_rows + 63) / 64, n32 = (s_rows + 31) / 32;
-  if (type != T_Q6_K && r2 * n64 >= 2 * cus) return {2, 2, n64};
+  if (type != T_Q6_K && r2 * n64 >= 2 * cus) return {type == T_Q8_0 ? 1 : 2, 2, n64};  // (Q8_0: as in an expert's down)
   return {r2 * n32 >= cus ? 2 : 1, 1, n32};
 }
 
@@ -974,7 +996,7 @@ hipError_t launch_plain_t(hipStream_t st, const F16Args &a, const Split &sp) {
   }
   const PlainShape p = plain_shape(T, a.rows, a.s_rows);
   if constexpr (T != T_Q6_K) {
-    if (p.nt == 2) return launch_t<T, 2, 2, 2>(st, a, p.blocks, sp);
+    if (p.nt == 2) return launch_t<T, 2, T == T_Q8_0 ? 1 : 2, 2>(st, a, p.blocks, sp);
   }
   if (p.rt == 2) return launch_t<T, 2, 2, 1>(st, a, p.blocks, sp);
   return launch_t<T, 2, 1, 1>(st, a, p.blocks, sp);

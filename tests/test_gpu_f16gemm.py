@@ -28,8 +28,8 @@ def _matmul(ctx, t, w, rows, cols, x):
 
 
 def _bound(t, w64, x, cols):
-    """Largest error of the sum of products: the pieces (2^-23 of each x, 2^-40
-    of the row's largest) and one fp32 rounding per 8 products of partial sums
+    """Largest error of the sum of products: the pieces (2^-23 of each x; 2^-17
+    of 2^-24 of the row's largest is more than they leave of small ones) and one fp32 rounding per 8 products of partial sums
     no larger than sum |w x| (Q4_K: of the scale and the minimum term apart, at
     most 8 times that for these blocks: |d sc q| + |dmin m| <= 7 * max |w| of
     the sub-block, its rms at least max / 4)."""
@@ -60,6 +60,32 @@ def test_plain_rows(ctx, t, rows, cols, S):
     assert np.all(np.abs(got - ref) <= _bound(t, w64, x, cols) + 1e-45)
     n = np.linalg.norm(ref, axis=1)
     assert np.all(np.linalg.norm(got - ref, axis=1) <= 1e-6 * n)
+
+
+# an element 2^24 above the others whose weights are all zero: what is left of
+# the sums keeps f32's bits (one and two token tiles; Q4_K's minimum term)
+@pytest.mark.parametrize("t,S", [(Q4_K, 70), (Q4_K, 1100), (Q6_K, 70), (Q8_0, 70), (Q8_0, 1100)])
+def test_small_elements_beside_a_large_one_keep_their_bits(ctx, t, S):
+    from oracle import pyoracle as orc
+
+    rows, cols = 8192, 512
+    w = random_blocks(t, rows, cols, seed=9)
+    b = w.reshape(rows, -1)
+    if t == Q8_0:
+        b[:, 2 + 7] = 0
+    elif t == Q4_K:  # the first sub-block's minimum and the element's nibble
+        b[:, 4 + 4] &= 0xC0
+        b[:, 16 + 7] &= 0xF0
+    else:  # q = 32
+        b[:, 7] &= 0xF0
+        b[:, 128 + 7] = (b[:, 128 + 7] & 0xFC) | 2
+    x = np.random.default_rng(S).standard_normal((S, cols)).astype(np.float32)
+    x[:, 7] = 2.0 ** 24
+    w64 = orc.dequant(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    assert not w64[:, 7].any()
+    ref = x[:, 8:].astype(np.float64) @ w64[:, 8:].T + x[:, :7].astype(np.float64) @ w64[:, :7].T
+    got = _matmul(ctx, t, w, rows, cols, x)
+    assert np.all(np.linalg.norm(got - ref, axis=1) <= 1e-6 * np.linalg.norm(ref, axis=1))
 
 
 @pytest.mark.parametrize("t", [Q4_K, Q6_K, Q8_0])
