@@ -854,20 +854,20 @@ namespace {
 // (lane l: chain l of each), 8 row tiles by 4 token tiles per work-group, so
 // that an element read from LDS is used TQ times; one logit per 16 lanes reads
 // two floats per FMA and is bound by that (1777 tokens by 128 rows of 2048:
-// 180-200 us; 4 x 4 tiles 60 us). Columns are staged 256 at a time, chain-major
+// 175 us; 2 x 2 tiles 44 us; 4 x 4 tiles, a quarter of the work-groups, 50 us and
+// behind 2 x 2 at every size measured). Columns are staged 256 at a time, chain-major
 // (element 8c + l at l * 36 + c: a lane reads four steps of its chain as 16
 // bytes, eight lanes 128 different bytes of the banks), the next chunk's loads
 // in flight meanwhile. A logit in dot_f32 order keeps the odd steps (its second
 // set of chains) in a second sum; row tiles without one skip that.
 // d % 256 == 0, 16-byte aligned rows, s_rows >= 4, not quant::dot order.
 constexpr int kRtChain = 36;  // a chain's 32 steps of a chunk and 4 words apart
-template <int TQ>
 __global__ void __launch_bounds__(256) k_router_tile(const float *__restrict__ W, int32_t E, int64_t d,
                                                      const float *__restrict__ X, int64_t S,
                                                      float *__restrict__ logits, int32_t nlog, int qkind,
                                                      int8_t *__restrict__ xq, float *__restrict__ xd,
                                                      int32_t *__restrict__ xs) {
-  constexpr int TE = 8 * TQ, TT = 4 * TQ, NL = (TE + TT) / 4;  // 16-byte loads per thread and chunk
+  constexpr int TQ = 2, TE = 8 * TQ, TT = 4 * TQ, NL = (TE + TT) / 4;  // 16-byte loads per thread and chunk
   __shared__ __attribute__((aligned(16))) float L[TE + TT][8 * kRtChain];
   if ((int32_t)blockIdx.x >= nlog) {  // the int8 rows of x, as in k_router_logits
     const int lane = threadIdx.x & 63;
@@ -984,22 +984,17 @@ hipError_t launch_router_logits(hipStream_t st, const float *router, int32_t n_e
                 n_expert, d, x, s_rows, logits, qdot ? 1 : 0, (int32_t)blocks, qkind, xq, xd, xs);
     return hipGetLastError();
   }
-  // Tiles of 4 x 4 or 2 x 2 logits per 8 lanes, where they still give about a
-  // work-group per CU, or one per two; below that the chains of single logits
-  // run at once on more CUs.
+  // Tiles of 2 x 2 logits per 8 lanes from about a work-group per two CUs; below
+  // that the chains of single logits run at once on more CUs. us, those ->
+  // tiles: 128 rows of 2048 by 64 tokens (64 work-groups) 9.6 -> 14.2, by 96 (96)
+  // 13.4 -> 14.6, by 128 (128) 15.5 -> 14.9, by 300 (304) 34.5 -> 17.6; 256 rows
+  // of 4096 by 48 (96) 22.0 -> 26.1, by 64 (128) 27.9 -> 26.3, by 1024 388 -> 90.
   if (!qdot && d % 256 == 0 && (((uintptr_t)router | (uintptr_t)x) & 15) == 0) {
-    const int64_t b4 = (s_rows + 15) / 16 * ((n_expert + 31) / 32), b2 = (s_rows + 7) / 8 * ((n_expert + 15) / 16);
-    if (b2 + qblocks <= (int64_t)INT32_MAX && n_expert > 8) {
-      if (b4 >= 200) {
-        KMOE_LAUNCH(k_router_tile<4>, dim3((unsigned)(b4 + qblocks)), dim3(256), 0, st, router, n_expert, d, x, s_rows,
-                    logits, (int32_t)b4, qkind, xq, xd, xs);
-        return hipGetLastError();
-      }
-      if (b2 >= 96) {
-        KMOE_LAUNCH(k_router_tile<2>, dim3((unsigned)(b2 + qblocks)), dim3(256), 0, st, router, n_expert, d, x, s_rows,
-                    logits, (int32_t)b2, qkind, xq, xd, xs);
-        return hipGetLastError();
-      }
+    const int64_t tiles = (s_rows + 7) / 8 * ((n_expert + 15) / 16);
+    if (tiles + qblocks <= (int64_t)INT32_MAX && n_expert > 8 && tiles >= 128) {
+      KMOE_LAUNCH(k_router_tile, dim3((unsigned)(tiles + qblocks)), dim3(256), 0, st, router, n_expert, d, x, s_rows,
+                  logits, (int32_t)tiles, qkind, xq, xd, xs);
+      return hipGetLastError();
     }
   }
   const int64_t blocks = (s_rows + 3) / 4 * ((n_expert + 3) / 4);
