@@ -329,11 +329,21 @@ __device__ __forceinline__ void unpack(const Raw<T> &w, int64_t st, int64_t nb, 
   for (int s = 0; s < 8; ++s) o[s] = __builtin_bit_cast(h8, u32x4{r[s][0], r[s][1], r[s][2], r[s][3]});
 }
 
+// The lane's number, read where it is used: a register held for it over the K
+// loop would spill others (the down product's two by two tiles: 2 registers, 181
+// us at 1777 Qwen3-shaped tokens, 165 without).
+__device__ __forceinline__ uint32_t lane_here() {
+  uint32_t all = 0xffffffffu;
+  asm volatile("" : "+s"(all));
+  return __builtin_amdgcn_mbcnt_hi(all, __builtin_amdgcn_mbcnt_lo(all, 0));
+}
+
 // The 8 minimums of a Q4_K superblock, times 32, as the MFMA's B operand (the K
 // halves: against the sums' hi and lo pieces).
 __device__ __forceinline__ h8 mins_operand(const u32x4 &hd) {
   h8 o;
-  const float f = (threadIdx.x & 32) ? 32.0f * kLo : 32.0f;
+  // 32 in the lower lanes, 32 * kLo in the upper ones
+  const float f = __builtin_bit_cast(float, 0x42000000u - (lane_here() >> 5) * (12u << 23));
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     int sA, mA, sB, mB;
@@ -533,7 +543,7 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
   };
   // Q4_K: the superblock's sums of tokens 32w .. 32w+31 by wave w < NT
   uint32_t ssrc = 0;
-  if constexpr (T == T_Q4_K)
+  if constexpr (T == T_Q4_K && MODE == 0)
     ssrc = (uint32_t)(src_row(32 * (wave % NT) + (lane >> 1)) * a.x.sums_stride) + 16 * (lane & 1);
   // LDS offset of this lane's A piece of K step s: aoff ^ 32s
   const int aoff = 256 * l32 + 16 * (hh ^ (l32 & 15));
@@ -664,9 +674,16 @@ __global__ void __launch_bounds__(256, 2) k_f16_gemm(F16Args a) {
       load_x(next, st + 1);
       if constexpr (T == T_Q4_K) {
         uint32_t o = ssrc;
-        asm volatile("" : "+v"(o));
+        const uint8_t *sb = (const uint8_t *)a.x.sums;
+        if constexpr (MODE == 0) {
+          asm volatile("" : "+v"(o));
+        } else {  // contiguous rows: formed here
+          const uint32_t l = lane_here(), t = 32 * (wave % NT) + (l >> 1), last = (uint32_t)(nbt - 1);
+          o = (t < last ? t : last) * (uint32_t)a.x.sums_stride + 16 * (l & 1);
+          sb += (p0 + tok0) * a.x.sums_stride;
+        }
         if (!odd && wave < NT)
-          lds_dma16((const uint8_t *)a.x.sums + 32 * (int64_t)(st >> 1) + o, next + NP * PLANE + ADS + wave * 1024);
+          lds_dma16(sb + 32 * (int64_t)(st >> 1) + o, next + NP * PLANE + ADS + wave * 1024);
       }
     }
     if constexpr (T == T_Q4_K && !INT) {  // y -= dmin * sum_j m_j S_j, once per superblock
