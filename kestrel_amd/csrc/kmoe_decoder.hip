@@ -424,7 +424,7 @@ __device__ __forceinline__ void attn_quant_group(const float *os, int group, int
 // many chunks are resident: eight chunks per round trip with m and l read
 // again for each, and one work-group per CU (f32 copies of K, V and q held in
 // 300 registers), took 38.5 us for one row of 16 heads of 128 at 3001
-// positions; this merge with three work-groups per CU 21 us (4096 positions
+// positions; this merge with three work-groups per CU 19.8 us (4096 positions
 // 49.6 -> 32.2; 8 rows of 16 heads over 4 at 1008 positions 25.0 -> 16.8).
 template <int HD>
 __device__ __forceinline__ void attn_merge(const float *pb, int nch, int lane, float *__restrict__ out, float *os) {

@@ -437,12 +437,14 @@ __device__ __forceinline__ bool find_block(const F16Args &a, int rblocks, int la
 // Two work-groups per CU (256 registers per lane): one unpacks while the
 // other's MFMAs run.
 // Measured on MI355X against the bf16-split and fp32 kernels (us, with the
-// split and reduction kernels): Qwen3 shape, 1777 tokens, gate/up 1195 -> 290,
-// down 680 -> 175; Q4_K 4096x4096 by 512 rows 184 -> 68; DeepSeek-V2-Lite
-// shape, 203 tokens, gate/up 293 -> 137, Q8_0 down 180 -> 83, shared Q6_K down
-// 278 -> 63. Its MFMAs run a third of the time; the rest is the weights' load
-// requests (32 lines per instruction), the unpacking and the short K loops'
-// ends. Error against 64 bits: 3.1e-7 -> 1.8e-7 (Q4_K matrix).
+// split and reduction kernels): Qwen3 shape, 1777 tokens, gate/up 1195 -> 308,
+// down 680 -> 187; Q4_K 4096x4096 by 512 rows 184 -> 66; DeepSeek-V2-Lite
+// shape, 203 tokens, gate/up 293 -> 143, Q8_0 down 180 -> 79, shared Q6_K down
+// 278 -> 32. Its MFMAs run 29% of the time (counted); the rest is the weights'
+// load requests (a row per lane: 32 lines per instruction), the unpacking and
+// the short K loops' ends. Error against 64 bits: 3.1e-7 -> 1.7e-7 (Q4_K
+// matrix). No form spills but Q8_0 gate/up by two token tiles (24 registers; 64
+// experts of 1408 by 2048, 1777 tokens 1118 us per layer, one tile 1371).
 //
 // INT: int8 activation rows (the int8 path, quant.rs:262-281) as one exact f16
 // piece. The MFMAs' sums are integers below 2^24 (Q4_K: 128 * 15*63 * 127 per
