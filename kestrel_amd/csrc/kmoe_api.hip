@@ -129,20 +129,30 @@ bool f16_plain(int t, int64_t rows, int64_t cols, int64_t s_rows) {
 // -> 350, 86 tokens 369 -> 369, 128 tokens 420 -> 385, 1777 tokens 2696 -> 1961.
 // Q4_K has int8 matrix-core kernels with the same arithmetic and bits. They pass
 // over an expert's rows 128 at a time in one work-group per 128 weight rows, so
-// a ragged layer waits for its fullest expert; below one token tile they read
-// the weights once with less work. All experts there -> those of more than 32
-// rows here: Qwen3 shape (Zipf 1.1) 200 tokens 240 -> 186, 1777 tokens 1241 ->
-// 602, evenly routed 300 tokens 202 -> 207, 1024 tokens 390 -> 430, 2048 tokens
-// 645 -> 669; 32 experts of 1536 by 2048, even, 400 tokens 167 -> 171, 2048
-// tokens 542 -> 530, Zipf 1.1, 400 tokens 292 -> 216, 1200 tokens 744 -> 387.
-// Wider parts fill the chip with one expert's work-groups: 32 of 1536 by 4096,
-// 512 tokens even 349 -> 379, Zipf 1 411 -> 419; 16 of 4096 by 2048, 512 tokens
-// even 332 -> 419, Zipf 1 404 -> 442; Mixtral shape 512 tokens 984 -> 1172.
-// In calls of few tokens the launches decide: Qwen3 shape 48 tokens 139 -> 148,
-// 64 tokens 144 -> 150, 96 tokens 168 -> 160.
-constexpr int kF16IntRows = 33, kF16IntTokens = 96;
-int f16_int(int t, int64_t d, int64_t F, int64_t S, int64_t slots, int64_t max_active) {
-  if (t == KMOE_Q4_K) return d * F <= (int64_t)8 << 20 && S >= kF16IntTokens ? kF16IntRows : 0;
+// a ragged layer waits for its fullest expert, and f16 takes the experts that
+// are fuller than the rest: of more than half as many rows again as the average
+// (an evenly routed layer has none, and splitting it between the two halves
+// what each can spread over the chip: 128 experts of 768 by 2048, 512 tokens 375
+// us split at 32 rows, 307 so). Where the average is at most 20, the int8
+// streaming kernel takes experts of up to 32 rows and f16 the others; from an
+// average of 105 most experts need a second pass there and f16 takes all above
+// one token tile. All experts there -> this: Qwen3 shape (Zipf 1.1) 200 tokens
+// 240 -> 188, 512 tokens 400 -> 276, 1777 tokens 1241 -> 602, evenly routed 300
+// tokens 202 -> 208, 1024 tokens 390 -> 403, 1777 tokens 565 -> 592; 32 experts of
+// 1536 by 2048, even, 900 tokens 303 -> 281, 2048 tokens 542 -> 530, Zipf 1.1,
+// 1200 tokens 744 -> 390. Few experts of few rows stay: there the launches that
+// find nothing show (32 experts, even, 128 tokens 102 -> 108, 700 tokens 230 ->
+// 238), as in calls of few tokens (Qwen3 shape 64 tokens 144 -> 150, 96 tokens
+// 168 -> 158). Wider parts fill the chip with one expert's work-groups: 32 of 1536
+// by 4096, 512 tokens even 349 -> 379, Zipf 1 411 -> 419; 16 of 4096 by 2048, 512
+// tokens even 332 -> 419, Zipf 1 404 -> 442; Mixtral shape 512 tokens 984 -> 1172.
+constexpr int64_t kF16IntRows = 33, kF16IntTokens = 96, kF16IntFull = 105;
+int f16_int(int t, int64_t E, int64_t d, int64_t F, int64_t S, int64_t slots, int64_t max_active) {
+  if (t == KMOE_Q4_K) {
+    const int64_t avg = slots / E;
+    if (d * F > (int64_t)8 << 20 || S < kF16IntTokens || (E < 64 && avg < kF16IntFull)) return 0;
+    return (int)(avg >= kF16IntFull || avg <= 20 ? kF16IntRows : std::max(kF16IntRows, avg + avg / 2 + 1));
+  }
   return slots >= (t == KMOE_Q6_K ? 16 : 8) * max_active ? 1 : 0;
 }
 // Expert layers, gate/up (whole layer, us): Mixtral shape 48 tokens 411 -> 488,
@@ -1757,7 +1767,7 @@ static int moe_ffn(kmoe_ctx *c, uint32_t layer, const float *h, int64_t S, float
                       const int32_t *qs, uint8_t *scratch, float *o, int lo, const BlockDbg *g) -> int {
     const bool mm = mfma && t == KMOE_Q4_K && moe_mfma_supported(rows, cols);
     int hi = (int)S;
-    const int f16 = regime == KMOE_REGIME_INT8 && (mm || t != KMOE_Q4_K) ? f16_int(t, d, F, S, slots, max_active) : 0;
+    const int f16 = regime == KMOE_REGIME_INT8 && (mm || t != KMOE_Q4_K) ? f16_int(t, E, d, F, S, slots, max_active) : 0;
     if (f16) {
       const int from = f16 > lo ? f16 : lo;
       const hipError_t e = timed(c, mode ? "moe_down_i8_f16" : "moe_gate_up_i8_f16", [&]() {

@@ -281,7 +281,7 @@ def test_capture_of_a_mixed_layer_keeps_the_int8_rows(ctx, dt):
 # oracle's, and the down product is within the roundings of its join. Rows past
 # one chain of roundings (17 superblocks), one and two token tiles.
 @pytest.mark.parametrize("gt,dt,E,S,F", [(Q6_K, Q6_K, 3, 60, 4352), (Q8_0, Q6_K, 6, 130, 512), (Q4_K, Q8_0, 3, 60, 4352),
-                                         (Q4_K, Q4_K, 4, 150, 4352), (Q6_K, Q8_0, 5, 33, 384)])
+                                         (Q4_K, Q4_K, 4, 240, 4352), (Q6_K, Q8_0, 5, 33, 384)])
 def test_int8_regime_down_is_the_exact_integers(ctx, gt, dt, E, S, F):
     import torch
     from oracle import pyoracle as orc
