@@ -138,7 +138,7 @@ bool f16_plain(int t, int64_t rows, int64_t cols, int64_t s_rows) {
 // average of 105 most experts need a second pass there and f16 takes all above
 // one token tile. All experts there -> this: Qwen3 shape (Zipf 1.1) 200 tokens
 // 240 -> 188, 512 tokens 400 -> 276, 1777 tokens 1241 -> 602, evenly routed 300
-// tokens 202 -> 208, 1024 tokens 390 -> 403, 1777 tokens 565 -> 592; 32 experts of
+// tokens 202 -> 208, 1024 tokens 390 -> 403, 2048 tokens 645 -> 672; 32 experts of
 // 1536 by 2048, even, 900 tokens 303 -> 281, 2048 tokens 542 -> 530, Zipf 1.1,
 // 1200 tokens 744 -> 390. Few experts of few rows stay: there the launches that
 // find nothing show (32 experts, even, 128 tokens 102 -> 108, 700 tokens 230 ->
