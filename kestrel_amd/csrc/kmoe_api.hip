@@ -207,6 +207,7 @@ struct kmoe_ctx {
   uint8_t *pws = nullptr;
   size_t pws_size = 0;
   bool pws_captured = false, pws_used = false, pws_wait = false;
+  hipStream_t pws_stream = nullptr;  // of the last use outside a capture
   hipEvent_t pws_event = nullptr;
   std::vector<void *> pws_retired;
   // last moe_ffn routing (pointers into ws) and its sizes
@@ -649,19 +650,26 @@ uint8_t *pieces(kmoe_ctx *c, size_t need) {
     c->pws = (uint8_t *)p;
     c->pws_size = sz;
   }
-  if (cap) c->pws_captured = true;
-  else if (c->pws_wait && hipStreamWaitEvent(c->stream, c->pws_event, 0) != hipSuccess) return nullptr;
-  else c->pws_wait = false;
+  if (cap) {
+    c->pws_captured = true;
+    return c->pws;
+  }
+  if (c->pws_wait && hipStreamWaitEvent(c->stream, c->pws_event, 0) != hipSuccess) {
+    (void)hipGetLastError();
+    return nullptr;
+  }
+  c->pws_wait = false;
   c->pws_used = true;
+  c->pws_stream = c->stream;
   return c->pws;
 }
 
-// The stream is about to change: what uses the pieces on the old one is marked.
+// The stream is about to change: the last use of the pieces is marked on its own.
 void leave_stream(kmoe_ctx *c, hipStream_t next) {
-  if (next == c->stream || !c->pws_used || capturing(c->stream) || capturing(next)) return;
+  if (!c->pws_used || next == c->pws_stream || capturing(c->pws_stream) || capturing(next)) return;
   DeviceGuard g(c->device);
   if ((!c->pws_event && hipEventCreateWithFlags(&c->pws_event, hipEventDisableTiming) != hipSuccess) ||
-      hipEventRecord(c->pws_event, c->stream) != hipSuccess) {
+      hipEventRecord(c->pws_event, c->pws_stream) != hipSuccess) {
     (void)hipGetLastError();  // no such stream any more
     return;
   }
